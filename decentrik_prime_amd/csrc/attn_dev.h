@@ -99,6 +99,26 @@ __device__ __forceinline__ void dma16(const void* src, unsigned lds) {
       : "memory");
 }
 
+// The same with a wave-uniform 64-bit base and a 32-bit byte offset per lane: one address register
+// per lane and no vector address arithmetic from tile to tile.
+__device__ __forceinline__ void dma16s(uint64_t base, unsigned off, unsigned lds) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "global_load_lds_dwordx4 %2, %3\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "s"(lds), "v"(off), "s"(base)
+      : "memory");
+}
+
+// A wave-uniform 64-bit value in scalar registers.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) |
+         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)v);
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmem() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -114,6 +134,37 @@ __device__ __forceinline__ f16x8 read_col8_sw(const f16* tile, int p, int col) {
   const int r = p + ((lane & 15) >> 2), c = col + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
   const f16x4 lo = read_tr(tile + sw_off(r, c)), hi = read_tr(tile + sw_off(r + 8, c));
   return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
+// The operand reads of a tile by LDS byte address.  The swizzle only flips chunk bits, so every
+// operand of a tile is a lane's base address with a constant XORed into it (plus a constant row
+// offset): K operand of sub-step s of rows 0..31 (+ 32 rows: 8192 bytes on) at kaddr ^ 32 s, and
+// the transposed columns of head block hb at vaddr ^ 64 hb (rows + 8: ^ 64 (hb ^ 2), 2048 on).
+typedef __attribute__((address_space(3))) const char lds_char;
+__device__ __forceinline__ f16x8 lds_read8(unsigned addr, int off) {
+  return *reinterpret_cast<__attribute__((address_space(3))) const f16x8*>((lds_char*)(size_t)addr + off);
+}
+__device__ __forceinline__ f16x4 lds_read_tr(unsigned addr, int off) {
+  return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) i16x4*)((lds_char*)(size_t)addr + off)));
+}
+// this lane's base for lds_read8 (row c = lane % 32, columns 8 (lane / 32) .. + 7) and for
+// lds_read_tr (see read_col8_sw: rows 4 (lane / 32) + lane % 16 / 4)
+__device__ __forceinline__ unsigned row_base(int lane) {
+  return (unsigned)(sw_off(lane & 31, 8 * (lane >> 5)) * 2);
+}
+__device__ __forceinline__ unsigned col_base(int lane) {
+  return (unsigned)(sw_off(4 * (lane >> 5) + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2);
+}
+__device__ __forceinline__ f16x8 lds_col8(unsigned caddr, int hb, int off) {
+  const f16x4 lo = lds_read_tr(caddr ^ (unsigned)(64 * hb), off);
+  const f16x4 hi = lds_read_tr(caddr ^ (unsigned)(64 * (hb ^ 2)), off + 2048);
+  return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+// keeps the compiler from holding every XORed address in a register of its own across the loop
+__device__ __forceinline__ unsigned fresh(unsigned a) {
+  asm volatile("" : "+v"(a));
+  return a;
 }
 
 // 2^x on the hardware exponential (v_exp_f32); arguments here are <= 0 (scores minus their row

@@ -8,19 +8,32 @@ namespace {
 
 // forward (solution/k_attn.py:40-83): one workgroup per (block of kBM queries, query head), 8
 // waves: wave w takes queries 32 (w % 4) .. + 31 of the block and the key tiles t with
-// t % 2 == w / 4, so two waves share each SIMD and each walks half of the block's tiles (the
-// causal blocks walk 2 to 8 tiles of 64 keys).  The two halves' softmax states (running maximum,
-// sum, O) are merged through LDS at the end.  Measured on MI355X at 4 x 512 tokens against 4
-// waves each walking every tile (one wave per SIMD): 19.7 -> 18.5 us.
+// t % 2 == w / 4, so two waves share each SIMD and each walks half of the block's tiles.  The two
+// halves' softmax states (running maximum, sum, O) are merged through LDS at the end.
+//
+// Bound: per tile of 64 keys a wave has 32 MFMAs (1024 clocks of its SIMD's matrix core), 48 LDS
+// operand reads and about 130 VALU instructions (32 of them quarter-rate exponentials).  One
+// after the other these ran at a quarter of the matrix rate, with both waves of a SIMD in the same
+// phase after every barrier.  So the scores of the wave's next tile are computed beside the
+// exponentials of the current one (S(t + 2) needs nothing of tile t), and the K ring runs a
+// pair of tiles ahead of the V ring.
 constexpr int kFThreads = 512;
 constexpr int kFLoads = kTileHalves / 8 / kFThreads;   // DMA instructions per operand per lane: 2
 
+// max over the two lanes l, l ^ 32 (the two key halves of one query)
+__device__ __forceinline__ float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __restrict__ out,
-                                                             float* __restrict__ lse) {
+                                                             float* __restrict__ lse, int n_blocks) {
+  // every head of a block before the next block, the table from its end: within a sequence the
+  // longest walks start first, so that no long block is left to run alone at the end
+  const int h = blockIdx.x % a.nq;
   int64_t s0;
   int seqlen, mstart;
-  if (!block_of(a, blockIdx.x, &s0, &seqlen, &mstart)) return;
-  const int h = blockIdx.y;
+  if (!block_of(a, n_blocks - 1 - (int)blockIdx.x / a.nq, &s0, &seqlen, &mstart)) return;
   const int lane = threadIdx.x & 63, hl = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int qw = wave & 3, kg = wave >> 2;   // query group, key-tile parity
@@ -34,32 +47,38 @@ __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __
   f32x16 oacc[kHD / 32];
 #pragma unroll
   for (int hb = 0; hb < kHD / 32; ++hb) oacc[hb] = zero16();
-  float m_i = -1.0e30f, l_i = 0.0f;
+  float m_i = -1.0e30f, l_i = 0.0f;   // l_i: this lane's half of the keys (joined at the end)
   const int hi = mstart + kBM < seqlen ? mstart + kBM : seqlen;
   const int n_tiles = (hi + kBN - 1) / kBN;
   const int n_pairs = (n_tiles + 1) / 2;
-  const f16* kbase = a.qkv + s0 * ROW + (int64_t)(a.nq + kvh) * kHD;
-  const f16* vbase = a.qkv + s0 * ROW + (int64_t)(a.nq + a.nkv + kvh) * kHD;
-  // tile t into stage t % 4: instruction i of wave w fills the stage's chunks (8 i + w) 64 + lane,
-  // row q / 16 (rows past the sequence read its last row: finite, and masked to p = 0)
-  auto issue = [&](int t) {
-    const int st = t % kFwdStages;
+  const uint64_t kbase = uniform64((uint64_t)(a.qkv + s0 * ROW + (int64_t)(a.nq + kvh) * kHD));
+  const uint64_t vbase = kbase + (uint64_t)a.nkv * kHD * sizeof(f16);
+  // tile pair u (tiles 2 u, 2 u + 1; tiles past the last: none) of one operand into stages t % 4:
+  // instruction i of wave w fills the stage's chunks (8 i + w) 64 + lane, row 32 i + r0 (rows past
+  // the sequence read its last row: finite, and masked to p = 0).  A row's offset inside its
+  // tile fits 32 bits: the host refuses head counts whose rows reach 2^32 / 64 bytes.
+  const int r0 = 4 * wave + (lane >> 4);
+  const unsigned rowb = (unsigned)(ROW * (int64_t)sizeof(f16));
+  const unsigned chunk = (unsigned)(((lane & 15) ^ swz16(r0)) << 4);
+  auto issue = [&](uint64_t base, f16* ring, int u) {
 #pragma unroll
-    for (int i = 0; i < kFLoads; ++i) {
-      const int q = (8 * i + wave) * 64 + lane, r = q >> 4;
-      const int row = t * kBN + r < seqlen ? t * kBN + r : seqlen - 1;
-      const int64_t src = (int64_t)row * ROW + (((q & 15) ^ swz16(r)) << 3);
-      const int dst = st * kTileHalves + (8 * i + wave) * 512;
-      dma16(kbase + src, __builtin_amdgcn_readfirstlane(lds_addr(Ks + dst)));
-      dma16(vbase + src, __builtin_amdgcn_readfirstlane(lds_addr(Vs + dst)));
+    for (int b = 0; b < 2; ++b) {
+      const int t = 2 * u + b;
+      if (t >= n_tiles) continue;
+      const uint64_t tb = base + (uint64_t)(t * kBN) * rowb;
+      const int last = seqlen - 1 - t * kBN;
+#pragma unroll
+      for (int i = 0; i < kFLoads; ++i) {
+        const int r = 32 * i + r0 < last ? 32 * i + r0 : last;
+        const int dst = (t % kFwdStages) * kTileHalves + (8 * i + wave) * 512;
+        dma16s(tb, (unsigned)r * rowb + chunk, __builtin_amdgcn_readfirstlane(lds_addr(ring + dst)));
+      }
     }
   };
-  // tile pair u = tiles 2 u, 2 u + 1: pair 0 now, pair 1 after the query loads
-  issue(0);
-  if (n_tiles > 1) issue(1);
+  issue(kbase, Ks, 0);
   // this lane's query row as the B operand (rows past the sequence: zeros).  Loaded at a clamped
   // row unconditionally and selected at once, so the compiler's wait for these loads stands here
-  // (it then also covers pair 0, issued above) and not inside the loop.
+  // (it then also covers the first K pair, issued above) and not inside the loop.
   f16x8 qf[kHD / 16];
   {
     const f16* qrow = a.qkv + (s0 + (mval ? m : mstart)) * ROW + h * kHD + 8 * hl;
@@ -73,91 +92,145 @@ __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __
     for (int s = 0; s < kHD / 16; ++s) qf[s] = mval ? qf[s] : zero8();
   }
   wait_vmem<0>();
-  if (n_tiles > 2) issue(2);
-  if (n_tiles > 3) issue(3);
+  issue(vbase, Vs, 0);
+  issue(kbase, Ks, 1);
   __syncthreads();
-  for (int u = 0; u < n_pairs; ++u) {
-    const int t = 2 * u + kg;
-    if (t < n_tiles) {
-      const f16* Kt = Ks + (t % kFwdStages) * kTileHalves;
-      const f16* Vt = Vs + (t % kFwdStages) * kTileHalves;
-      const int n0 = t * kBN;
-      // S^T = K Q^T: keys kb * 32 + (row of the result), queries on the lanes
-      f32x16 sc[2];
-      sc[0] = sc[1] = zero16();
+  const unsigned krow = lds_addr(Ks) + row_base(lane), vcol = lds_addr(Vs) + col_base(lane);
+  // S^T = K Q^T of tile t: keys kb * 32 + (row of the result), queries on the lanes
+  auto scores = [&](f32x16 (&sc)[2], int t) {
+    const unsigned ka = fresh(krow + (unsigned)((t % kFwdStages) * kTileHalves * 2));
+    sc[0] = sc[1] = zero16();
 #pragma unroll
-      for (int s = 0; s < kHD / 16; ++s)
+    for (int s = 0; s < kHD / 16; ++s)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          sc[kb] = mfma(*reinterpret_cast<const f16x8*>(Kt + sw_off(kb * 32 + c, 16 * s + 8 * hl)),
-                        qf[s], sc[kb]);
-      // keys past this lane's query (or the sequence end) masked: key n = n0 + off + 4 (l / 32)
-      // is kept iff off <= min(m, seqlen - 1) - n0 - 4 (l / 32).  Only tiles that reach the
-      // block's first query hold masked keys (the test is uniform).  A lane can see a tile whose
-      // keys are all masked before any kept key (this wave skips every other tile): its masked
-      // probabilities are set to 0 below rather than computed from the running maximum.
-      const int lim = (m < seqlen - 1 ? m : seqlen - 1) - n0 - 4 * hl;
-      const bool diag = n0 + kBN > mstart;
-      if (diag) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            sc[kb][v] = kb * 32 + 8 * (v >> 2) + (v & 3) <= lim ? sc[kb][v] : -1.0e30f;
-      }
-      // the row maximum of the raw scores, scaled once (the scaling is monotonic)
-      float mx = -1.0e30f;
+      for (int kb = 0; kb < 2; ++kb)
+        sc[kb] = mfma(lds_read8(ka ^ (unsigned)(32 * s), kb * 32 * kHD * 2), qf[s], sc[kb]);
+  };
+  f32x16 sc[2], sn[2];
+  if (kg < n_tiles) scores(sc, kg);
+  wait_vmem<0>();
+  __syncthreads();
+  // tile t, whose scores are in sc: its softmax and O^T += V^T P^T, beside the scores of tile
+  // t + 2 into sn when there is one.  DIAG: the tile may hold masked keys (past this lane's query or
+  // the sequence end): key n = n0 + off + 4 (l / 32) is kept iff
+  // off <= min(m, seqlen - 1) - n0 - 4 (l / 32).  A lane can see a tile whose keys are all masked
+  // before any kept key (this wave skips every other tile): masked probabilities are set to 0
+  // rather than computed from the running maximum.
+  auto tile = [&](int t, bool more, f32x16 (&sc)[2], f32x16 (&sn)[2], auto diag_c) {
+    constexpr bool DIAG = decltype(diag_c)::value;
+    const unsigned va = fresh(vcol + (unsigned)((t % kFwdStages) * kTileHalves * 2));
+    const int lim = (m < seqlen - 1 ? m : seqlen - 1) - t * kBN - 4 * hl;
+    if constexpr (DIAG) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sc[kb][v]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      // m_i is the reference point of l_i and O, not the exact running maximum: it moves (and O
-      // and l are rescaled) only when some lane's maximum exceeds it by more than 2^8, so p =
-      // 2^(s * qk_scale - m_i) stays below 256 and the rescale, a read-modify-write of all of O,
-      // runs on the first tile and rarely after.  The decision is per wave (uniform branch).
-      const float mt = __fmul_rn(mx, a.qk_scale);
-      if (__builtin_amdgcn_ballot_w64(mt > m_i + 8.0f) != 0) {
-        const float m_new = fmaxf(m_i, mt);
-        const float alpha = ex2(__fsub_rn(m_i, m_new));
-        l_i = __fmul_rn(l_i, alpha);
-        m_i = m_new;
-#pragma unroll
-        for (int hb = 0; hb < kHD / 32; ++hb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) oacc[hb][v] = __fmul_rn(oacc[hb][v], alpha);
-      }
-      float rs = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const bool kept = !diag || kb * 32 + 8 * (v >> 2) + (v & 3) <= lim;
-          const float p = kept ? ex2(__builtin_fmaf(sc[kb][v], a.qk_scale, -m_i)) : 0.0f;
-          sc[kb][v] = p;
-          rs = __fadd_rn(rs, p);
-        }
-      rs = __fadd_rn(rs, __shfl_xor(rs, 32));
-      l_i = __fadd_rn(l_i, rs);
-      // O^T += V^T P^T over the tile's 64 keys, 16 per step
-#pragma unroll
-      for (int tt = 0; tt < kBN / 16; ++tt) {
-        const int kb = tt >> 1, i0 = 8 * (tt & 1);
-        f16x8 pf;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pf[j] = (f16)sc[kb][i0 + j];
-#pragma unroll
-        for (int hb = 0; hb < kHD / 32; ++hb)
-          oacc[hb] = mfma(read_col8_sw(Vt, 16 * tt + 4 * hl, hb * 32), pf, oacc[hb]);
-      }
+        for (int v = 0; v < 16; ++v)
+          sc[kb][v] = kb * 32 + 8 * (v >> 2) + (v & 3) <= lim ? sc[kb][v] : -1.0e30f;
     }
-    // pair u + 1 landed (this wave's loads) and visible to every wave, and every wave is done
-    // with pair u's stages, which then receive pair u + 2
+    // the row maximum of the raw scores, scaled once (the scaling is monotonic)
+    float mx = -1.0e30f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sc[kb][v]);
+    mx = half_max(mx);
+    // m_i is the reference point of l_i and O, not the exact running maximum: it moves (and O
+    // and l are rescaled) only when some lane's maximum exceeds it by more than 2^8, so p =
+    // 2^(s * qk_scale - m_i) stays below 256 and the rescale, a read-modify-write of all of O,
+    // runs on the first tile and rarely after.  The decision is per wave (uniform branch).
+    const float mt = __fmul_rn(mx, a.qk_scale);
+    if (__builtin_amdgcn_ballot_w64(mt > m_i + 8.0f) != 0) {
+      const float m_new = fmaxf(m_i, mt);
+      const float alpha = ex2(__fsub_rn(m_i, m_new));
+      l_i = __fmul_rn(l_i, alpha);
+      m_i = m_new;
+#pragma unroll
+      for (int hb = 0; hb < kHD / 32; ++hb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[hb][v] = __fmul_rn(oacc[hb][v], alpha);
+    }
+    if (!DIAG || more) scores(sn, t + 2);
+    float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    f16x8 pf[kBN / 16];   // P^T as the B operand: keys 16 tt .. + 15
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float p = ex2(__builtin_fmaf(sc[kb][v], a.qk_scale, -m_i));
+        if constexpr (DIAG) p = kb * 32 + 8 * (v >> 2) + (v & 3) <= lim ? p : 0.0f;
+        rs[v & 3] = __fadd_rn(rs[v & 3], p);
+        pf[2 * kb + (v >> 3)][v & 7] = (f16)p;
+      }
+    l_i = __fadd_rn(l_i, __fadd_rn(__fadd_rn(rs[0], rs[1]), __fadd_rn(rs[2], rs[3])));
+    // O^T += V^T P^T over the tile's 64 keys, 16 per step
+#pragma unroll
+    for (int tt = 0; tt < kBN / 16; ++tt)
+#pragma unroll
+      for (int hb = 0; hb < kHD / 32; ++hb)
+        oacc[hb] = mfma(lds_col8(va, hb, 16 * tt * kHD * 2), pf[tt], oacc[hb]);
+    // the next tile's scores spread over the exponentials, their operands read four MFMAs ahead;
+    // then O, its operands four MFMAs (eight reads) ahead
+    if constexpr (!DIAG) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int i = 0; i < 12; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+      }
+    } else {
+      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 200, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+  };
+  using Diag = std::integral_constant<bool, true>;
+  using Full = std::integral_constant<bool, false>;
+  // V of pair u and K of pair u + 1 are in LDS; K of pair u + 2 goes where pair u's was (its
+  // scores are done), V of pair u + 1 where pair u - 1's was
+  auto fetch = [&](int u) {
+    issue(vbase, Vs, u + 1);
+    issue(kbase, Ks, u + 2);
+  };
+  // the loads of fetch(u) have landed and are visible, and every wave is done with pair u's V and
+  // pair u + 1's K
+  auto next = [&]() {
     wait_vmem<0>();
     __syncthreads();
-    if (2 * u + 4 < n_tiles) issue(2 * u + 4);
-    if (2 * u + 5 < n_tiles) issue(2 * u + 5);
+  };
+  // pairs whose tiles both lie before the block's first query (no masked key) and have a next
+  // tile, two at a time so that the two score buffers need no copies; then the last ones
+  int full = mstart / (2 * kBN);
+  if (full > (n_tiles - 2) / 2) full = (n_tiles - 2) / 2;
+  if (full < 0) full = 0;
+  int u = 0;
+  for (; u + 2 <= full; u += 2) {
+    fetch(u);
+    tile(2 * u + kg, true, sc, sn, Full{});
+    next();
+    fetch(u + 1);
+    tile(2 * u + 2 + kg, true, sn, sc, Full{});
+    next();
   }
+  for (; u < n_pairs; ++u) {
+    fetch(u);
+    const int t = 2 * u + kg;
+    if (t < n_tiles) tile(t, t + 2 < n_tiles, sc, sn, Diag{});
+    sc[0] = sn[0];
+    sc[1] = sn[1];
+    next();
+  }
+  l_i = __fadd_rn(l_i, __shfl_xor(l_i, 32));
   // merge: the odd-tile wave of each query group hands its state (O lane-major, 16 KB per wave,
   // in the K stages; m and l in the V stages' last KB) to the even-tile wave, which combines
   // O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise, m = max(m0, m1).  Every stage is free after
@@ -229,8 +302,9 @@ extern "C" int dk_attn_fwd(const void* qkv, const int32_t* cu_seqlens, int32_t n
   if (n_blocks == 0) return 0;
   if (!out || !lse) return DK_ERR_INVALID;
   if (!dk_aligned(out, 16) || !dk_aligned(lse, 4)) return DK_ERR_ALIGN;
-  hipLaunchKernelGGL(attn_fwd_kernel, dim3((unsigned)n_blocks, (unsigned)nq), dim3(kFThreads), 0,
-                     stream, a, (f16*)out, lse);
+  if ((int64_t)n_blocks * nq > INT32_MAX) return DK_ERR_INVALID;   // one workgroup index
+  hipLaunchKernelGGL(attn_fwd_kernel, dim3((unsigned)(n_blocks * nq)), dim3(kFThreads), 0,
+                     stream, a, (f16*)out, lse, n_blocks);
   DK_CHECK_LAUNCH();
   return 0;
 }
