@@ -24,9 +24,65 @@ __global__ __launch_bounds__(kAThreads) void attn_delta_kernel(const f16* __rest
   if ((threadIdx.x & 15) == 0) delta[(int64_t)hh * n_tokens + t] = s;
 }
 
+// The tile ring of both backward kernels: a tile of two operands (kBN rows each) in one of four
+// LDS stages, filled by LDS DMA.  Wave w's instruction i fills chunks (4 i + w) 64 + lane of an
+// operand: row 16 i + 4 w + lane / 16, with a wave-uniform base per tile and a 32-bit offset per
+// lane; rows past `rows` (the rows left in the sequence, less one) read that row (finite, masked
+// to p = 0).
+constexpr int kBwdStages = 4;
+constexpr int kBwdLoads = kTileHalves / 8 / kAThreads;   // per operand per lane: 4
+constexpr unsigned kStageBytes = kTileHalves * 2;
+
+struct TileSource {
+  uint64_t base;      // first row of tile 0
+  unsigned rowb;      // bytes per row
+  unsigned off0;      // this lane's offset for instruction 0
+  unsigned chunk;     // this lane's (swizzled) chunk offset inside a row
+};
+__device__ __forceinline__ TileSource tile_source(const f16* base, int64_t row_halves, int wave,
+                                                  int lane) {
+  TileSource t;
+  t.base = uniform64((uint64_t)base);
+  t.rowb = (unsigned)(row_halves * (int64_t)sizeof(f16));
+  const int r0 = 4 * wave + (lane >> 4);
+  t.chunk = (unsigned)(((lane & 15) ^ swz16(r0)) << 4);
+  t.off0 = (unsigned)r0 * t.rowb + t.chunk;
+  return t;
+}
+__device__ __forceinline__ void tile_load(const TileSource& src, int64_t first_row, int rows,
+                                          const f16* stage, int wave) {
+  const uint64_t tb = src.base + (uint64_t)first_row * src.rowb;
+  const unsigned last = (unsigned)(rows < kBN ? rows : kBN) * src.rowb + src.chunk;
+#pragma unroll
+  for (int i = 0; i < kBwdLoads; ++i) {
+    const unsigned off = src.off0 + (unsigned)(16 * i) * src.rowb;
+    dma16s(tb, off < last ? off : last,
+           __builtin_amdgcn_readfirstlane(lds_addr(stage + (4 * i + wave) * 512)));
+  }
+}
+
+// A barrier that orders the LDS DMA waited for before it, without a wait for the operand reads in
+// flight (they are of stages that no load in flight touches).
+__device__ __forceinline__ void tile_barrier() {
+  wait_vmem<0>();
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Both backward kernels run one wave per SIMD (their accumulators and resident operands take most
+// of its 512 registers), so what hides a wave's latencies is its own instruction order: tile t's
+// step is 32 MFMAs of tile t + 1's two score products with one element of tile t's P and dS beside
+// each, then the MFMAs that consume P and dS.  Every operand read stands four to six MFMAs before
+// its use, also across the two phases and from step to step, and the one barrier of a step lies
+// between the phases: after it, tile t - 1's stage takes tile t + 3, and tile t + 2 is readable.
+// The order is held by scheduling barriers: left to itself the compiler waited for each operand
+// read right before its MFMA.
+constexpr int kAhead1 = 6, kAhead2 = 4;
+
 // dQ (solution/k_attn.py:142-182): one workgroup per (block of kBM queries, query head), key
-// tiles of kBN up to the diagonal, in the forward's four-stage K/V ring; the S^T and dP^T MFMAs of
-// tile t + 1 run beside the dS work of tile t
+// tiles of kBN up to the diagonal
 __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
                                          const f16* __restrict__ dout,
                                          const float* __restrict__ lse,
@@ -44,23 +100,17 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
 
   const int hi = mstart + kBM < seqlen ? mstart + kBM : seqlen;
   const int n_tiles = (hi + kBN - 1) / kBN;
-  const f16* kbase = a.qkv + s0 * ROW + (int64_t)(a.nq + kvh) * kHD;
-  const f16* vbase = a.qkv + s0 * ROW + (int64_t)(a.nq + a.nkv + kvh) * kHD;
-  constexpr int kLoads = kTileHalves / 8 / kAThreads;
-  auto issue = [&](int t, int st) {
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const int q = (4 * i + wave) * 64 + lane, r = q >> 4;
-      const int row = t * kBN + r < seqlen ? t * kBN + r : seqlen - 1;
-      const int64_t src = (int64_t)row * ROW + (((q & 15) ^ swz16(r)) << 3);
-      const int dst = st * kTileHalves + (4 * i + wave) * 512;
-      dma16(kbase + src, __builtin_amdgcn_readfirstlane(lds_addr(Ks + dst)));
-      dma16(vbase + src, __builtin_amdgcn_readfirstlane(lds_addr(Vs + dst)));
-    }
+  const TileSource ksrc = tile_source(a.qkv + s0 * ROW + (int64_t)(a.nq + kvh) * kHD, ROW, wave, lane);
+  const TileSource vsrc = tile_source(a.qkv + s0 * ROW + (int64_t)(a.nq + a.nkv + kvh) * kHD, ROW, wave, lane);
+  auto issue = [&](int t) {
+    if (t >= n_tiles) return;
+    const int st = t % kBwdStages;
+    tile_load(ksrc, t * kBN, seqlen - 1 - t * kBN, Ks + st * kTileHalves, wave);
+    tile_load(vsrc, t * kBN, seqlen - 1 - t * kBN, Vs + st * kTileHalves, wave);
   };
-  issue(0, 0);
-  if (n_tiles > 1) issue(1, 1);
-  if (n_tiles > 2) issue(2, 2);
+  issue(0);
+  issue(1);
+  issue(2);
   // this lane's query and dO rows and statistics, loaded at a clamped row and selected at once
   // (the compiler's wait for them stands here, not in the loop)
   f16x8 qf[kHD / 16], dof[kHD / 16];
@@ -90,78 +140,104 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
   f32x16 dqacc[kHD / 32];
 #pragma unroll
   for (int hb = 0; hb < kHD / 32; ++hb) dqacc[hb] = zero16();
-  // S^T = K Q^T and dP^T = V dO^T of the tile in stage st: keys kb * 32 + (row), queries on lanes
-  auto products = [&](f32x16 (&sacc)[2], f32x16 (&dpacc)[2], int st) {
-    const f16* Kt = Ks + st * kTileHalves;
-    const f16* Vt = Vs + st * kTileHalves;
-    sacc[0] = sacc[1] = dpacc[0] = dpacc[1] = zero16();
-#pragma unroll
-    for (int s = 0; s < kHD / 16; ++s)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int o = sw_off(kb * 32 + c, 16 * s + 8 * hl);
-        sacc[kb] = mfma(*reinterpret_cast<const f16x8*>(Kt + o), qf[s], sacc[kb]);
-        dpacc[kb] = mfma(*reinterpret_cast<const f16x8*>(Vt + o), dof[s], dpacc[kb]);
-      }
+  const unsigned krow = lds_addr(Ks) + row_base(lane), vrow = lds_addr(Vs) + row_base(lane);
+  const unsigned kcol = lds_addr(Ks) + col_base(lane);
+  // operand i of a tile's products: S^T = K Q^T and dP^T = V dO^T (keys kb * 32 + (row), queries
+  // on the lanes): sub-step i / 4, dP^T for i / 2 odd, key half i % 2
+  auto rd1 = [&](unsigned ka, unsigned va, int i) {
+    return lds_read8((((i >> 1) & 1) ? va : ka) ^ (unsigned)(32 * (i >> 2)), (i & 1) * 32 * kHD * 2);
   };
-  if (n_tiles > 2) wait_vmem<2 * kLoads>();
-  else wait_vmem<0>();
-  __syncthreads();
-  f32x16 sc[2], dc[2];
-  products(sc, dc, 0);
-  for (int t = 0; t < n_tiles; ++t) {
-    if (t + 3 < n_tiles) issue(t + 3, (t + 3) % kFwdStages);
-    const f16* Kt = Ks + (t % kFwdStages) * kTileHalves;
+  auto product = [&](f32x16 (&sacc)[2], f32x16 (&dpacc)[2], const f16x8& f, int i) {
+    const int s = i >> 2, kb = i & 1;
+    if ((i >> 1) & 1) dpacc[kb] = mfma(f, dof[s], s == 0 ? zero16() : dpacc[kb]);
+    else sacc[kb] = mfma(f, qf[s], s == 0 ? zero16() : sacc[kb]);
+  };
+  f16x8 fr[kAhead1];
+  // the wait for all three tiles costs no more than the query rows' own
+  tile_barrier();
+  f32x16 s_a[2], d_a[2], s_b[2], d_b[2];
+  {
+    const unsigned ka = fresh(krow), va = fresh(vrow);
+#pragma unroll
+    for (int i = 0; i < kAhead1; ++i) fr[i] = rd1(ka, va, i);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      product(s_a, d_a, fr[i % kAhead1], i);
+      if (i + kAhead1 < 32) fr[i % kAhead1] = rd1(ka, va, i + kAhead1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const unsigned ka1 = fresh(krow + kStageBytes), va1 = fresh(vrow + kStageBytes);
+#pragma unroll
+    for (int i = 0; i < kAhead1; ++i) fr[i] = rd1(ka1, va1, i);
+  }
+  auto step = [&](int t, f32x16 (&sc)[2], f32x16 (&dc)[2], f32x16 (&sn)[2], f32x16 (&dn)[2],
+                  auto more_c) {
+    constexpr bool MORE = decltype(more_c)::value;   // tile t + 1 exists
     const int n0 = t * kBN;
-    f32x16 sn[2], dn[2];
-    products(sn, dn, (t + 1) % kFwdStages);
-    // P and dS^T = P (dP^T - delta).  Rows past the sequence have zero q, dO and delta, so their
-    // dS is zero whatever P is; keys past a query or the sequence are masked only on the tiles
-    // that reach this wave's first query (a wave-uniform test): key n = n0 + off + 4 (l / 32) is
-    // kept iff off <= min(m, seqlen - 1) - n0 - 4 (l / 32).  The exponential is computed for
-    // every score and then selected (a conditional exponential becomes a branch).
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        sc[kb][v] = ex2(__builtin_fmaf(sc[kb][v], a.qk_scale, -lse_m));
+    // keys past a query or the sequence are masked only on the tiles that reach this wave's first
+    // query (a wave-uniform test): key n = n0 + off + 4 (l / 32) is kept iff
+    // off <= min(m, seqlen - 1) - n0 - 4 (l / 32); the others' probabilities come out as 0.
+    // Rows past the sequence have zero q, dO and delta, so their dS is zero whatever P is.
     if (n0 + kBN - 1 > mstart + 32 * wave || n0 + kBN > seqlen) {
       const int lim = (m < seqlen - 1 ? m : seqlen - 1) - n0 - 4 * hl;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          sc[kb][v] = kb * 32 + 8 * (v >> 2) + (v & 3) <= lim ? sc[kb][v] : 0.0f;
+          sc[kb][v] = kb * 32 + 8 * (v >> 2) + (v & 3) <= lim ? sc[kb][v] : -1.0e30f;
     }
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) sc[kb][v] = __fmul_rn(sc[kb][v], __fsub_rn(dc[kb][v], dl_m));
+    const unsigned nst = (unsigned)((t + 1) % kBwdStages) * kStageBytes;
+    const unsigned ka = fresh(krow + nst), va = fresh(vrow + nst);
+    const unsigned kc = fresh(kcol + (unsigned)(t % kBwdStages) * kStageBytes);
+    auto rd2 = [&](int i) { return lds_col8(kc, i & 3, 16 * (i >> 2) * kHD * 2); };
+    f16x8 dsf[kBN / 16], gr[kAhead2];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an operand read
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // an MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);   // VALU
+      if constexpr (MORE) {
+        product(sn, dn, fr[i % kAhead1], i);
+        if (i + kAhead1 < 32) fr[i % kAhead1] = rd1(ka, va, i + kAhead1);
+      }
+      const int kb = i >> 4, v = i & 15;
+      const float p = ex2(__builtin_fmaf(sc[kb][v], a.qk_scale, -lse_m));
+      dsf[2 * kb + (v >> 3)][v & 7] = (f16)__fmul_rn(p, __fsub_rn(dc[kb][v], dl_m));
+      if (i >= 32 - kAhead2) gr[i - (32 - kAhead2)] = rd2(i - (32 - kAhead2));
+      if constexpr (MORE) __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (MORE) {
+      tile_barrier();
+      issue(t + 3);
+    }
+    const unsigned nst2 = (unsigned)((t + 2) % kBwdStages) * kStageBytes;
+    const unsigned ka2 = fresh(krow + nst2), va2 = fresh(vrow + nst2);
     // dQ^T += K^T dS^T
 #pragma unroll
-    for (int tt = 0; tt < kBN / 16; ++tt) {
-      const int kb = tt >> 1, i0 = 8 * (tt & 1);
-      f16x8 dsf;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dsf[j] = (f16)sc[kb][i0 + j];
-#pragma unroll
-      for (int hb = 0; hb < kHD / 32; ++hb)
-        dqacc[hb] = mfma(read_col8_sw(Kt, 16 * tt + 4 * hl, hb * 32), dsf, dqacc[hb]);
+    for (int i = 0; i < 16; ++i) {
+      dqacc[i & 3] = mfma(gr[i % kAhead2], dsf[i >> 2], dqacc[i & 3]);
+      if (i + kAhead2 < 16) gr[i % kAhead2] = rd2(i + kAhead2);
+      // (past the last tile: a stale stage, never used)
+      if (MORE && i >= 16 - kAhead1) fr[i - (16 - kAhead1)] = rd1(ka2, va2, i - (16 - kAhead1));
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (t + 3 < n_tiles) wait_vmem<2 * kLoads>();
-    else wait_vmem<0>();
-    __syncthreads();
-    sc[0] = sn[0];
-    sc[1] = sn[1];
-    dc[0] = dn[0];
-    dc[1] = dn[1];
+  };
+  using More = std::integral_constant<bool, true>;
+  using Last = std::integral_constant<bool, false>;
+  int t = 0;
+  for (; t + 2 < n_tiles; t += 2) {
+    step(t, s_a, d_a, s_b, d_b, More{});
+    step(t + 1, s_b, d_b, s_a, d_a, More{});
   }
+  if (t + 1 < n_tiles) {
+    step(t, s_a, d_a, s_b, d_b, More{});
+    ++t;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      s_a[kb] = s_b[kb];
+      d_a[kb] = d_b[kb];
+    }
+  }
+  step(t, s_a, d_a, s_b, d_b, Last{});
+  __syncthreads();
   // the wave's 32 x 128 block of dQ staged in the (now free) tile ring, waves 0-1 in the K stages
   // and 2-3 in the V stages, then written back 16 bytes per lane, two whole 512-byte rows per
   // store instruction (stored from the registers, each instruction would cover 32 bytes of each
@@ -204,11 +280,8 @@ __device__ __forceinline__ void dma4(const void* src, unsigned lds) {
 // dK, dV per query head (solution/k_attn.py:97-139): one workgroup per (block of kBM keys, query
 // head), query tiles of kBN from the block's first key to the end of the sequence; fp32 partials
 // [N, NQ HD] that the QKV epilogue backward sums over each group of NQ / NKV heads.  The Q and dO
-// tiles and the tiles' lse and delta rows come through a four-stage LDS ring filled by LDS DMA
-// (swizzled rows as in the forward; the statistics by dword DMA, one lane per query, waves 0
-// and 1), and the S and dP MFMAs of tile t + 1 run beside the P / dS work of tile t.
-constexpr int kBwdStages = 4;
-
+// tiles and the tiles' lse and delta rows (by dword DMA, one lane per query, waves 0 and 1) come
+// through the four-stage ring.
 __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
                                            const f16* __restrict__ dout,
                                            const float* __restrict__ lse,
@@ -226,45 +299,24 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
   const int n = nstart + 32 * w + c;   // this lane's key
   const bool nval = n < seqlen && s0 + n < a.n_tokens;
 
-  const int n_tiles = nstart < seqlen ? (seqlen - nstart + kBN - 1) / kBN : 0;
-  const f16* qbase = a.qkv + s0 * ROW + (int64_t)h * kHD;
-  const f16* dbase = dout + s0 * OROW + (int64_t)h * kHD;
-  constexpr int kLoads = kTileHalves / 8 / kAThreads;   // per operand per lane: 4
-  // query tile t (queries nstart + 64 t ...) into stage st; rows past the sequence read its last
-  // row (finite, masked to p = 0); wave 0 also fetches the tile's lse, wave 1 its delta
-  auto issue = [&](int t, int st) {
-    const int m0 = nstart + t * kBN;
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const int q = (4 * i + wave) * 64 + lane, r = q >> 4;
-      const int row = m0 + r < seqlen ? m0 + r : seqlen - 1;
-      const int off = ((q & 15) ^ swz16(r)) << 3;
-      const int dst = st * kTileHalves + (4 * i + wave) * 512;
-      dma16(qbase + (int64_t)row * ROW + off, __builtin_amdgcn_readfirstlane(lds_addr(Qs + dst)));
-      dma16(dbase + (int64_t)row * OROW + off, __builtin_amdgcn_readfirstlane(lds_addr(Ds + dst)));
-    }
+  const int n_tiles = (seqlen - nstart + kBN - 1) / kBN;   // at least 1 (block_of)
+  const TileSource qsrc = tile_source(a.qkv + (s0 + nstart) * ROW + (int64_t)h * kHD, ROW, wave, lane);
+  const TileSource dsrc = tile_source(dout + (s0 + nstart) * OROW + (int64_t)h * kHD, OROW, wave, lane);
+  // query tile t (queries nstart + 64 t ...); wave 0 also fetches the tile's lse, wave 1 its delta
+  auto issue = [&](int t) {
+    if (t >= n_tiles) return;
+    const int st = t % kBwdStages, m0 = nstart + t * kBN;
+    tile_load(qsrc, t * kBN, seqlen - 1 - m0, Qs + st * kTileHalves, wave);
+    tile_load(dsrc, t * kBN, seqlen - 1 - m0, Ds + st * kTileHalves, wave);
     if (wave < 2) {
       const int qq = m0 + lane < seqlen ? m0 + lane : seqlen - 1;
       const float* src = (wave == 0 ? lse : delta) + (int64_t)h * a.n_tokens + s0 + qq;
       dma4(src, __builtin_amdgcn_readfirstlane(lds_addr(wave == 0 ? lse_s[st] : dl_s[st])));
     }
   };
-  // wait until at most `tiles` tiles of this wave's loads are in flight (waves 0 and 1 issue one
-  // more load per tile)
-  auto wait_tiles = [&](int tiles) {
-    if (wave < 2) {
-      if (tiles >= 2) wait_vmem<2 * (2 * kLoads + 1)>();
-      else if (tiles == 1) wait_vmem<2 * kLoads + 1>();
-      else wait_vmem<0>();
-    } else {
-      if (tiles >= 2) wait_vmem<2 * 2 * kLoads>();
-      else if (tiles == 1) wait_vmem<2 * kLoads>();
-      else wait_vmem<0>();
-    }
-  };
-  if (n_tiles > 0) issue(0, 0);
-  if (n_tiles > 1) issue(1, 1);
-  if (n_tiles > 2) issue(2, 2);
+  issue(0);
+  issue(1);
+  issue(2);
 
   // this lane's key and value rows as B operands, loaded at a clamped row and selected at once
   // (the compiler's wait for them stands here, not in the loop)
@@ -289,54 +341,50 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
   f32x16 dkacc[kHD / 32], dvacc[kHD / 32];
 #pragma unroll
   for (int hb = 0; hb < kHD / 32; ++hb) dkacc[hb] = dvacc[hb] = zero16();
-  // S = Q K^T and dP = dO V^T of the tile in stage st: queries qb * 32 + (row of the result),
-  // keys on the lanes
-  auto products = [&](f32x16 (&sacc)[2], f32x16 (&dpacc)[2], int st) {
-    const f16* Qt = Qs + st * kTileHalves;
-    const f16* Dt = Ds + st * kTileHalves;
-    sacc[0] = sacc[1] = dpacc[0] = dpacc[1] = zero16();
-#pragma unroll
-    for (int s = 0; s < kHD / 16; ++s)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        const int o = sw_off(qb * 32 + c, 16 * s + 8 * hl);
-        sacc[qb] = mfma(*reinterpret_cast<const f16x8*>(Qt + o), kf[s], sacc[qb]);
-        dpacc[qb] = mfma(*reinterpret_cast<const f16x8*>(Dt + o), vf[s], dpacc[qb]);
-      }
+  const unsigned qrow = lds_addr(Qs) + row_base(lane), drow = lds_addr(Ds) + row_base(lane);
+  const unsigned qcol = lds_addr(Qs) + col_base(lane), dcol = lds_addr(Ds) + col_base(lane);
+  // operand i of a tile's products S = Q K^T and dP = dO V^T (queries qb * 32 + (row of the
+  // result), keys on the lanes): sub-step i / 4, dP for i / 2 odd, query half i % 2
+  auto rd1 = [&](unsigned qa, unsigned da, int i) {
+    return lds_read8((((i >> 1) & 1) ? da : qa) ^ (unsigned)(32 * (i >> 2)), (i & 1) * 32 * kHD * 2);
   };
-  if (n_tiles > 0) {
-    wait_tiles(n_tiles > 2 ? 1 : 0);   // tiles 0 and 1 landed
-    __syncthreads();
+  auto product = [&](f32x16 (&sacc)[2], f32x16 (&dpacc)[2], const f16x8& f, int i) {
+    const int s = i >> 2, qb = i & 1;
+    if ((i >> 1) & 1) dpacc[qb] = mfma(f, vf[s], s == 0 ? zero16() : dpacc[qb]);
+    else sacc[qb] = mfma(f, kf[s], s == 0 ? zero16() : sacc[qb]);
+  };
+  // the statistics of rows 8 g + 4 (l / 32) + 0..3 of the tile in stage st (g = 0..7)
+  auto stat = [&](const float (*tab)[kBN], int st, int g) {
+    return *reinterpret_cast<const f32x4*>(&tab[st][8 * g + 4 * hl]);
+  };
+  f16x8 fr[kAhead1];
+  f32x4 ls[2], dl[2];
+  tile_barrier();
+  f32x16 s_a[2], d_a[2], s_b[2], d_b[2];
+  {
+    const unsigned qa = fresh(qrow), da = fresh(drow);
+#pragma unroll
+    for (int i = 0; i < kAhead1; ++i) fr[i] = rd1(qa, da, i);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      product(s_a, d_a, fr[i % kAhead1], i);
+      if (i + kAhead1 < 32) fr[i % kAhead1] = rd1(qa, da, i + kAhead1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const unsigned qa1 = fresh(qrow + kStageBytes), da1 = fresh(drow + kStageBytes);
+#pragma unroll
+    for (int i = 0; i < kAhead1; ++i) fr[i] = rd1(qa1, da1, i);
+    ls[0] = stat(lse_s, 0, 0);
+    dl[0] = stat(dl_s, 0, 0);
   }
-  f32x16 sc[2], dc[2];
-  if (n_tiles > 0) products(sc, dc, 0);
-  for (int t = 0; t < n_tiles; ++t) {
-    // stage (t + 3) % 4 held tile t - 1, whose last reader every wave finished before the
-    // barrier that ended iteration t - 1
-    if (t + 3 < n_tiles) issue(t + 3, (t + 3) % kBwdStages);
-    const int st = t % kBwdStages;
-    const int m0 = nstart + t * kBN;
-    // tile t + 1's products (past the last tile: a stale stage, never used)
-    f32x16 sn[2], dn[2];
-    products(sn, dn, (t + 1) % kBwdStages);
-    // the statistics of this lane's 32 queries of the tile: rows qb * 32 + 8 g + 4 (l / 32) + 0..3
-    f32x4 ls[2][4], ds[2][4];
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        ls[qb][g] = *reinterpret_cast<const f32x4*>(&lse_s[st][qb * 32 + 8 * g + 4 * hl]);
-        ds[qb][g] = *reinterpret_cast<const f32x4*>(&dl_s[st][qb * 32 + 8 * g + 4 * hl]);
-      }
-    // P, computed for every score and then selected (a conditional exponential becomes a branch).
+  auto step = [&](int t, f32x16 (&sc)[2], f32x16 (&dc)[2], f32x16 (&sn)[2], f32x16 (&dn)[2],
+                  auto more_c) {
+    constexpr bool MORE = decltype(more_c)::value;   // tile t + 1 exists
+    const int st = t % kBwdStages, m0 = nstart + t * kBN;
     // Keys past the sequence only reach rows of dK and dV that are not stored; queries before a
     // key or past the sequence are masked only on the tiles that hold such a query for this wave
-    // (a wave-uniform test): query q = m0 + off + 4 (l / 32) is kept iff lo <= off < hi.
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        sc[qb][v] = ex2(__builtin_fmaf(sc[qb][v], a.qk_scale, -ls[qb][v >> 2][v & 3]));
+    // (a wave-uniform test): query q = m0 + off + 4 (l / 32) is kept iff lo <= off < hi; the
+    // others' probabilities come out as 0.
     if (m0 < nstart + 32 * wave + 31 || m0 + kBN > seqlen) {
       const int lo = n - m0 - 4 * hl, hi = seqlen - m0 - 4 * hl;
 #pragma unroll
@@ -344,47 +392,71 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int off = qb * 32 + 8 * (v >> 2) + (v & 3);
-          sc[qb][v] = ((off >= lo) & (off < hi)) ? sc[qb][v] : 0.0f;
+          sc[qb][v] = ((off >= lo) & (off < hi)) ? sc[qb][v] : -1.0e30f;
         }
     }
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)   // dS
-        dc[qb][v] = __fmul_rn(sc[qb][v], __fsub_rn(dc[qb][v], ds[qb][v >> 2][v & 3]));
-    // the 32 products of tile t + 1 spread among this work
+    const unsigned nst = (unsigned)((t + 1) % kBwdStages) * kStageBytes;
+    const unsigned qa = fresh(qrow + nst), da = fresh(drow + nst);
+    const unsigned qc = fresh(qcol + (unsigned)st * kStageBytes), dc_ = fresh(dcol + (unsigned)st * kStageBytes);
+    auto rd2 = [&](int i) { return lds_col8((i & 1) ? qc : dc_, (i >> 1) & 3, 16 * (i >> 3) * kHD * 2); };
+    f16x8 pf[kBN / 16], dsf[kBN / 16], gr[kAhead2];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an operand read
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // an MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // VALU
+      if constexpr (MORE) {
+        product(sn, dn, fr[i % kAhead1], i);
+        if (i + kAhead1 < 32) fr[i % kAhead1] = rd1(qa, da, i + kAhead1);
+      }
+      const int qb = i >> 4, v = i & 15, g = i >> 2;
+      if ((i & 3) == 0 && g + 1 < 8) {
+        ls[(g + 1) & 1] = stat(lse_s, st, g + 1);
+        dl[(g + 1) & 1] = stat(dl_s, st, g + 1);
+      }
+      const float p = ex2(__builtin_fmaf(sc[qb][v], a.qk_scale, -ls[g & 1][i & 3]));
+      pf[2 * qb + (v >> 3)][v & 7] = (f16)p;
+      dsf[2 * qb + (v >> 3)][v & 7] = (f16)__fmul_rn(p, __fsub_rn(dc[qb][v], dl[g & 1][i & 3]));
+      if (i >= 32 - kAhead2) gr[i - (32 - kAhead2)] = rd2(i - (32 - kAhead2));
+      if constexpr (MORE) __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (MORE) {
+      tile_barrier();
+      issue(t + 3);
+    }
+    const unsigned nst2 = (unsigned)((t + 2) % kBwdStages) * kStageBytes;
+    const unsigned qa2 = fresh(qrow + nst2), da2 = fresh(drow + nst2);
     // dV += P^T dO, dK += dS^T Q over the tile's 64 queries, 16 per step
-    const f16* Qt = Qs + st * kTileHalves;
-    const f16* Dt = Ds + st * kTileHalves;
 #pragma unroll
-    for (int tt = 0; tt < kBN / 16; ++tt) {
-      const int qb = tt >> 1, i0 = 8 * (tt & 1);
-      f16x8 pf, dsf;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        pf[j] = (f16)sc[qb][i0 + j];
-        dsf[j] = (f16)dc[qb][i0 + j];
+    for (int i = 0; i < 32; ++i) {
+      const int hb = (i >> 1) & 3;
+      if (i & 1) dkacc[hb] = mfma(dsf[i >> 3], gr[i % kAhead2], dkacc[hb]);
+      else dvacc[hb] = mfma(pf[i >> 3], gr[i % kAhead2], dvacc[hb]);
+      if (i + kAhead2 < 32) gr[i % kAhead2] = rd2(i + kAhead2);
+      if constexpr (MORE) {
+        // (past the last tile: a stale stage, never used)
+        if (i >= 32 - kAhead1) fr[i - (32 - kAhead1)] = rd1(qa2, da2, i - (32 - kAhead1));
+        if (i == 28) ls[0] = stat(lse_s, (t + 1) % kBwdStages, 0);
+        if (i == 29) dl[0] = stat(dl_s, (t + 1) % kBwdStages, 0);
       }
-#pragma unroll
-      for (int hb = 0; hb < kHD / 32; ++hb) {
-        dvacc[hb] = mfma(pf, read_col8_sw(Dt, 16 * tt + 4 * hl, hb * 32), dvacc[hb]);
-        dkacc[hb] = mfma(dsf, read_col8_sw(Qt, 16 * tt + 4 * hl, hb * 32), dkacc[hb]);
-      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // tile t + 2 landed and visible to every wave, every wave done with stage t % 4
-    wait_tiles(t + 3 < n_tiles ? 1 : 0);
-    __syncthreads();
-    sc[0] = sn[0];
-    sc[1] = sn[1];
-    dc[0] = dn[0];
-    dc[1] = dn[1];
+  };
+  using More = std::integral_constant<bool, true>;
+  using Last = std::integral_constant<bool, false>;
+  int t = 0;
+  for (; t + 2 < n_tiles; t += 2) {
+    step(t, s_a, d_a, s_b, d_b, More{});
+    step(t + 1, s_b, d_b, s_a, d_a, More{});
   }
+  if (t + 1 < n_tiles) {
+    step(t, s_a, d_a, s_b, d_b, More{});
+    ++t;
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      s_a[qb] = s_b[qb];
+      d_a[qb] = d_b[qb];
+    }
+  }
+  step(t, s_a, d_a, s_b, d_b, Last{});
   // result register v of block hb: key 32 w + 8 (v / 4) + 4 (l / 32) + v % 4, column hb * 32 + c
 #pragma unroll
   for (int v = 0; v < 16; ++v) {

@@ -54,24 +54,25 @@ __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __
   const uint64_t kbase = uniform64((uint64_t)(a.qkv + s0 * ROW + (int64_t)(a.nq + kvh) * kHD));
   const uint64_t vbase = kbase + (uint64_t)a.nkv * kHD * sizeof(f16);
   // tile pair u (tiles 2 u, 2 u + 1; tiles past the last: none) of one operand into stages t % 4:
-  // instruction i of wave w fills the stage's chunks (8 i + w) 64 + lane, row 32 i + r0 (rows past
+  // instruction i of wave w fills the stage's chunks (8 i + w) 64 + lane (rows past
   // the sequence read its last row: finite, and masked to p = 0).  A row's offset inside its
   // tile fits 32 bits: the host refuses head counts whose rows reach 2^32 / 64 bytes.
-  const int r0 = 4 * wave + (lane >> 4);
   const unsigned rowb = (unsigned)(ROW * (int64_t)sizeof(f16));
-  const unsigned chunk = (unsigned)(((lane & 15) ^ swz16(r0)) << 4);
+  const unsigned chunk = (unsigned)(((lane & 15) ^ swz16(4 * wave + (lane >> 4))) << 4);
+  const unsigned off0 = (unsigned)(4 * wave + (lane >> 4)) * rowb + chunk;
   auto issue = [&](uint64_t base, f16* ring, int u) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const int t = 2 * u + b;
       if (t >= n_tiles) continue;
       const uint64_t tb = base + (uint64_t)(t * kBN) * rowb;
-      const int last = seqlen - 1 - t * kBN;
+      const int rows = seqlen - 1 - t * kBN;
+      const unsigned last = (unsigned)(rows < kBN ? rows : kBN) * rowb + chunk;   // kBN: none clamped
 #pragma unroll
       for (int i = 0; i < kFLoads; ++i) {
-        const int r = 32 * i + r0 < last ? 32 * i + r0 : last;
+        const unsigned off = off0 + (unsigned)(32 * i) * rowb;
         const int dst = (t % kFwdStages) * kTileHalves + (8 * i + wave) * 512;
-        dma16s(tb, (unsigned)r * rowb + chunk, __builtin_amdgcn_readfirstlane(lds_addr(ring + dst)));
+        dma16s(tb, off < last ? off : last, __builtin_amdgcn_readfirstlane(lds_addr(ring + dst)));
       }
     }
   };
