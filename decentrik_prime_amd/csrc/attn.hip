@@ -190,7 +190,8 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
     const unsigned ka = fresh(krow + nst), va = fresh(vrow + nst);
     const unsigned kc = fresh(kcol + (unsigned)(t % kBwdStages) * kStageBytes);
     auto rd2 = [&](int i) { return lds_col8(kc, i & 3, 16 * (i >> 2) * kHD * 2); };
-    f16x8 dsf[kBN / 16], gr[kAhead2];
+    Frag8 dsf[kBN / 16];
+    f16x8 gr[kAhead2];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
@@ -200,7 +201,8 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
       }
       const int kb = i >> 4, v = i & 15;
       const float p = ex2(__builtin_fmaf(sc[kb][v], a.qk_scale, -lse_m));
-      dsf[2 * kb + (v >> 3)][v & 7] = (f16)__fmul_rn(p, __fsub_rn(dc[kb][v], dl_m));
+      dc[kb][v] = __fmul_rn(p, __fsub_rn(dc[kb][v], dl_m));
+      if (i & 1) dsf[i >> 3].h[(i >> 1) & 3] = pinned(dc[kb][v - 1], dc[kb][v]);
       if (i >= 32 - kAhead2) gr[i - (32 - kAhead2)] = rd2(i - (32 - kAhead2));
       if constexpr (MORE) __builtin_amdgcn_sched_barrier(0);
     }
@@ -213,7 +215,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
     // dQ^T += K^T dS^T
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      dqacc[i & 3] = mfma(gr[i % kAhead2], dsf[i >> 2], dqacc[i & 3]);
+      dqacc[i & 3] = mfma(gr[i % kAhead2], dsf[i >> 2].get(), dqacc[i & 3]);
       if (i + kAhead2 < 16) gr[i % kAhead2] = rd2(i + kAhead2);
       // (past the last tile: a stale stage, never used)
       if (MORE && i >= 16 - kAhead1) fr[i - (16 - kAhead1)] = rd1(ka2, va2, i - (16 - kAhead1));
@@ -399,7 +401,8 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
     const unsigned qa = fresh(qrow + nst), da = fresh(drow + nst);
     const unsigned qc = fresh(qcol + (unsigned)st * kStageBytes), dc_ = fresh(dcol + (unsigned)st * kStageBytes);
     auto rd2 = [&](int i) { return lds_col8((i & 1) ? qc : dc_, (i >> 1) & 3, 16 * (i >> 3) * kHD * 2); };
-    f16x8 pf[kBN / 16], dsf[kBN / 16], gr[kAhead2];
+    Frag8 pf[kBN / 16], dsf[kBN / 16];
+    f16x8 gr[kAhead2];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
@@ -412,9 +415,12 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
         ls[(g + 1) & 1] = stat(lse_s, st, g + 1);
         dl[(g + 1) & 1] = stat(dl_s, st, g + 1);
       }
-      const float p = ex2(__builtin_fmaf(sc[qb][v], a.qk_scale, -ls[g & 1][i & 3]));
-      pf[2 * qb + (v >> 3)][v & 7] = (f16)p;
-      dsf[2 * qb + (v >> 3)][v & 7] = (f16)__fmul_rn(p, __fsub_rn(dc[qb][v], dl[g & 1][i & 3]));
+      sc[qb][v] = ex2(__builtin_fmaf(sc[qb][v], a.qk_scale, -ls[g & 1][i & 3]));
+      dc[qb][v] = __fmul_rn(sc[qb][v], __fsub_rn(dc[qb][v], dl[g & 1][i & 3]));
+      if (i & 1) {
+        pf[i >> 3].h[(i >> 1) & 3] = pinned(sc[qb][v - 1], sc[qb][v]);
+        dsf[i >> 3].h[(i >> 1) & 3] = pinned(dc[qb][v - 1], dc[qb][v]);
+      }
       if (i >= 32 - kAhead2) gr[i - (32 - kAhead2)] = rd2(i - (32 - kAhead2));
       if constexpr (MORE) __builtin_amdgcn_sched_barrier(0);
     }
@@ -428,8 +434,8 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
       const int hb = (i >> 1) & 3;
-      if (i & 1) dkacc[hb] = mfma(dsf[i >> 3], gr[i % kAhead2], dkacc[hb]);
-      else dvacc[hb] = mfma(pf[i >> 3], gr[i % kAhead2], dvacc[hb]);
+      if (i & 1) dkacc[hb] = mfma(dsf[i >> 3].get(), gr[i % kAhead2], dkacc[hb]);
+      else dvacc[hb] = mfma(pf[i >> 3].get(), gr[i % kAhead2], dvacc[hb]);
       if (i + kAhead2 < 32) gr[i % kAhead2] = rd2(i + kAhead2);
       if constexpr (MORE) {
         // (past the last tile: a stale stage, never used)

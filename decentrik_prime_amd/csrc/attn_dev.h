@@ -167,6 +167,21 @@ __device__ __forceinline__ unsigned fresh(unsigned a) {
   return a;
 }
 
+// Two values rounded to fp16, computed where they stand: without the empty asm the compiler sinks
+// the work down to its use, past the scheduling barriers that interleave it with MFMAs.
+__device__ __forceinline__ f16x2 pinned(float lo, float hi) {
+  f16x2 h = f16x2{(f16)lo, (f16)hi};
+  asm volatile("" : "+v"(h));
+  return h;
+}
+// elements i - 1, i (i odd) of 16-bit operands of 8
+struct Frag8 {
+  f16x2 h[4];
+  __device__ __forceinline__ f16x8 get() const {
+    return f16x8{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+  }
+};
+
 // 2^x on the hardware exponential (v_exp_f32); arguments here are <= 0 (scores minus their row
 // maximum or log-sum-exp), results below the normal range flush to zero.
 __device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
