@@ -56,11 +56,40 @@ struct GemmParams {
   int64_t rope_cols;
 };
 
-// Runs the GEMM of `p` (fp16 weight p.w16) on the 256 x 256-tile kernel when the shape suits it:
-// output columns a multiple of 256, K a multiple of 64, and either at least one tile per CU, or
-// (LINEAR, at least 4 row tiles, K of 4096 or more) a split-K that fills the CUs, whose fp32
-// partials need hgemm_workspace bytes of `ws`, or 128 x 128 tiles that fill at least half the
-// CUs.  p.side's workgroups (if any) join the launch.  Returns kHgemmDeclined without launching
+constexpr int kBK = 64;   // K per step of both kernels
+
+// Launch plan of w4gemm.hip's kernel: tile shape and split-K factor.  256 CUs.  A 128-row tile's workgroup needs
+// 76.8 KB of LDS (60 KB at 64 columns) and at most 128 VGPRs, so two share a CU (512 slots).
+// (256 x 128 tiles, one workgroup per CU, measured slower at these shapes and are not
+// planned.)  Shapes with fewer tiles than slots split K (at least 8 steps per split) so that about
+// 768 workgroups run: the fp32 partial tiles cost one extra pass over the output in the second
+// launch, so short K (under 64 steps) prefers narrower tiles and splits only below 256 tiles.
+struct Plan {
+  int bm, bn, splits;
+  int64_t tiles;
+};
+
+inline Plan plan_for(int64_t M, int64_t N, int64_t K, int epi) {
+  const int64_t nk = K / kBK;
+  const int64_t mt128 = (M + 127) / 128;
+  Plan pl{128, 128, 1, mt128 * (N / 128)};
+  if (N % 128 != 0) pl = {128, 64, 1, mt128 * (N / 64)};
+  if (epi != EPI_LINEAR || pl.tiles >= 512) return pl;
+  if (pl.bn == 128 && nk < 64) pl = {128, 64, 1, mt128 * (N / 64)};
+  if ((pl.tiles < 256 && nk >= 16) || (pl.tiles < 512 && nk >= 64)) {
+    int64_t s = (768 + pl.tiles - 1) / pl.tiles;
+    if (s > nk / 8) s = nk / 8;
+    if (s > 8) s = 8;
+    if (s >= 2) pl.splits = (int)s;
+  }
+  return pl;
+}
+
+// Runs the GEMM of `p` (fp16 weight p.w16) on hgemm.hip's kernels when the shape suits them: output
+// columns a multiple of 256, K a multiple of 64, and at least one 256 x 256 tile per CU or one of
+// the smaller plans (128 x 128 tiles, 128 x 256 tiles, 256 x 256 tiles, the last two with or
+// without split K, whose fp32 partials need hgemm_workspace bytes of `ws`) estimated faster than
+// w4gemm.hip's kernel.  p.side's workgroups (if any) join the launch.  Returns kHgemmDeclined without launching
 // anything otherwise, a HIP error code, or 0.
 constexpr int kHgemmDeclined = -1000;
 // W4: the weight read as packed NF4 (p.packed, p.qabs, p.scale2, p.offset2, p.code2, p.nf4; no

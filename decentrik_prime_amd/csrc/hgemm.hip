@@ -27,6 +27,9 @@
 // The DMA writes 64 consecutive 16-byte chunks per instruction, so the swizzle is applied to the
 // global addresses each lane loads.
 //
+// Fewer tiles than CUs run as 128 x 128 tiles, 128 x 256 tiles (hgemm_mid_kernel) or 256 x 256
+// tiles, the last two with or without split K, by an estimate of each plan's time (hplan_small).
+//
 // Tiles are dealt M-fastest inside each XCD's contiguous run of workgroups.  When the tile count
 // leaves a last round at most half full, those last tiles run as four 128 x 128 sub-tiles each
 // (8 waves of 32 x 64), so the final round is short instead of mostly idle; in the SwiGLU
@@ -50,12 +53,15 @@ namespace {
 
 typedef float f32x8_t __attribute__((ext_vector_type(8)));
 
-constexpr int kBK = 64;                      // K per step
 constexpr int kStages = 2;                   // LDS stages
 constexpr int kThreads = 512;
 constexpr int kTile = 256;
 constexpr int kStageHalves = kTile * kBK;    // one operand of one stage: 32 KB
 constexpr int kEpiScratch = 16384;           // bytes of LDS per wave for the epilogue
+constexpr int kMidRows = 128;                // rows of a 128 x 256 tile
+constexpr int kMidStages = 3;
+constexpr int kMidHalves = kMidStages * (kMidRows + kTile) * kBK;   // its LDS: 144 KB
+static_assert(8 * kEpiScratch <= kMidHalves * 2, "epilogue scratch of a 128 x 256 tile");
 
 // Epilogue scratch of a wave with TN 32-column blocks per strip: the staged strip (32 rows of
 // 32 TN + 4 floats) plus the keep-mask and LoRA A slices (1536 bytes each).
@@ -112,6 +118,14 @@ __device__ __forceinline__ f16x4 read_tr(const f16* p) {
 // for the first).
 __device__ __forceinline__ int swz_k(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
 __device__ __forceinline__ int swz_n(int k) { return (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)); }
+
+// Workgroup t of n consecutive ones, dealt to the 8 XCDs round-robin, as an index that gives each
+// XCD a contiguous run (the first n % 8 of them one more).  Measured on MI355X with split K over
+// 128 x 256 tiles at M = 853: 252 workgroups whose runs were not contiguous 53 us, 34 with runs.
+__device__ __forceinline__ int xcd_run(int t, int n) {
+  const int o = t & 7, q = n >> 3, r = n & 7;
+  return o * q + (o < r ? o : r) + (t >> 3);
+}
 
 // The fused epilogue of one wave's TM x TN blocks of 32 x 32 results, whose top-left output
 // element is (mw0, nw0).  A block is four 16 x 16 v_mfma_f32_16x16x32_f16 results: register v of
@@ -462,8 +476,11 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
                                           int nk, float* part, f16* As, f16* Bs,
                                           const float* w4tab) {
   constexpr int SA = BM * kBK, SB = BN * kBK;   // halves per stage of A and of W
-  static_assert(NST * SA <= kStages * kStageHalves && NST * SB <= kStages * kStageHalves &&
-                (NST & (NST - 1)) == 0 && NST >= 2, "LDS stages");
+  constexpr bool MID = BM == 128 && BN == 256;   // As and Bs are one array (hgemm_mid_kernel)
+  static_assert(NST >= 2 && (MID ? NST * (SA + SB) <= kMidHalves
+                                 : NST * SA <= kStages * kStageHalves &&
+                                       NST * SB <= kStages * kStageHalves), "LDS stages");
+  auto stage_of = [](int kt) { return (NST & (NST - 1)) == 0 ? kt & (NST - 1) : kt % NST; };
   constexpr bool SPEC = BM == 128 && BN == 128 && !W4 && !TRANS;   // waves split by role
 
   constexpr int NCW = SPEC ? 4 : 8;         // computing waves
@@ -637,7 +654,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
         __syncthreads();
         if (kt + NST < nk)
 #pragma unroll
-          for (int d = 0; d < LOADS; ++d) issue(kt + NST, kt & (NST - 1), d);
+          for (int d = 0; d < LOADS; ++d) issue(kt + NST, stage_of(kt), d);
       }
       // the second 32-row strip of computing wave w - NCW, handed over through LDS (below), and
       // its epilogue: every wave finishes one 32 x 64 strip, as in the 8-wave 128 x 128 tile
@@ -772,7 +789,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
 #pragma unroll
   for (int j = 0; j < TN16; ++j) read_b(0, 0, j, 0);
   for (int kt = 0; kt < nk; ++kt) {
-    const int st = kt & (NST - 1);
+    const int st = stage_of(kt);
     W4Piece w4_after;
     if constexpr (W4) {
       // step kt + NST + 1's packed piece (clamped at the end: loaded, never written)
@@ -793,7 +810,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
     else if (!SPEC) wait_loads((nk - 1 < kt + NST - 1 ? nk - 1 : kt + NST - 1) - (kt + 1));
     __syncthreads();
     const bool more = kt + 1 < nk;
-    const int st1 = (kt + 1) & (NST - 1);
+    const int st1 = stage_of(kt + 1);
     const bool refill = !SPEC && kt + NST < nk;
     if constexpr (W4) {
       if (refill) w4_write(st);
@@ -861,10 +878,14 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
     return;
   }
   // the epilogue scratch: 16 KB per wave, waves 0-3 in the A stages, 4-7 in the W stages
-  uint8_t* escr = reinterpret_cast<uint8_t*>(wave < 4 ? As : Bs) + (wave & 3) * kEpiScratch;
+  // (one array of a 128 x 256 tile: eight times 16 KB from its start)
+  auto scratch_of = [&](int w) {
+    return MID ? reinterpret_cast<uint8_t*>(As) + w * kEpiScratch
+               : reinterpret_cast<uint8_t*>(w < 4 ? As : Bs) + (w & 3) * kEpiScratch;
+  };
+  uint8_t* escr = scratch_of(wave);
   // the partner wave: the other 64-column half of the same rows (rotary epilogue)
-  const int pw = wave ^ 1;
-  const uint8_t* pscr = reinterpret_cast<const uint8_t*>(pw < 4 ? As : Bs) + (pw & 3) * kEpiScratch;
+  const uint8_t* pscr = scratch_of(wave ^ 1);
   static_assert(WAVES_N % 2 == 0, "partner waves share rows");
   wave_epilogue<TRANS, EPI, TM, TN>(p, acc, m0 + wm * WM, n0 + wn * WN, escr, pscr);
 }
@@ -965,15 +986,7 @@ void hgemm_kernel(GemmParams p, int main_tiles, int tail_wgs, int persist) {
   const int qbase = kQuartersFirst ? 0 : main_tiles;  // first quarter workgroup
   int b = blockIdx.x;
   if (b >= fbase && b < fbase + main_tiles) {
-    // workgroups are dealt to the 8 XCDs round-robin (workgroup i to XCD i % 8): give each XCD a
-    // contiguous run of tiles.  XCD x's full-tile workgroups are first, first + 8, ... from the
-    // first index at or past fbase that it receives.
-    if ((main_tiles & 7) == 0) {
-      const int x = b & 7, first = fbase + ((x - fbase) & 7);
-      b = x * (main_tiles >> 3) + ((b - first) >> 3);
-    } else {
-      b -= fbase;
-    }
+    b = xcd_run(b - fbase, main_tiles);
     // split-K: the splits are the slowest index, so an XCD's run covers neighbouring tiles of
     // one K range, which share A and W slices in its L2
     const int tiles = main_tiles / p.splits;
@@ -1000,8 +1013,7 @@ void hgemm_kernel(GemmParams p, int main_tiles, int tail_wgs, int persist) {
       m0 = (int64_t)((x % gm) * bm) * kTile + 128 * qm;
       n0 = (int64_t)(main_tiles / p.tiles_m + (x / gm) * bn) * kTile + 128 * qn;
     } else {
-      int u = t;
-      if ((tail_wgs & 7) == 0 && (qbase & 7) == 0) u = (u & 7) * (tail_wgs >> 3) + (u >> 3);
+      const int u = xcd_run(t, tail_wgs);
       const int parent = main_tiles + u / 4, quarter = u % 4;
       m0 = (int64_t)(parent % p.tiles_m) * kTile + 128 * (quarter & 1);
       n0 = (int64_t)(parent / p.tiles_m) * kTile + 128 * (quarter >> 1);
@@ -1011,21 +1023,59 @@ void hgemm_kernel(GemmParams p, int main_tiles, int tail_wgs, int persist) {
   }
 }
 
-// Split-K, second launch: one wave per 32 x 32 block of a 256 x 256 tile (64 per tile) sums the
-// block's split partials in split order (fixed, so the result is deterministic) and runs the
-// epilogue on it.  The kernel boundary orders it after every partial store.
+// The same GEMM on 128 x 256 tiles (8 waves of 64 x 64, three LDS stages): half the rows per tile,
+// for row counts that 256-row tiles pad by much or deal badly over the CUs, with split K for every
+// LINEAR shape that has fewer tiles than CUs.  The p.sums.wgs and p.side.wgs workgroups after the
+// tiles carry work as in hgemm_kernel.
 template <bool TRANS, int EPI>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void hgemm_mid_kernel(GemmParams p, int tiles_wgs) {
+  __shared__ __attribute__((aligned(1024))) f16 S[kMidHalves];
+  static_assert(side_dequant_lds <= kMidHalves * 2 && colsum_lds_bytes<16>() <= kMidHalves * 2,
+                "carried work in the kernel's LDS");
+  int b = blockIdx.x;
+  if (b >= tiles_wgs) {
+    b -= tiles_wgs;
+    if constexpr (TRANS && EPI == EPI_LINEAR) {
+      if (b < p.sums.wgs) {
+        colsum_run<16>(p.sums.jobs, p.sums.rows, colsum_block_of(b, p.sums.wgs, tiles_wgs),
+                       reinterpret_cast<uint8_t*>(S));
+        return;
+      }
+      b -= p.sums.wgs;
+    }
+    side_dequant(p.side, b, reinterpret_cast<uint8_t*>(S));
+    return;
+  }
+  // each XCD a contiguous run of tiles, M-fastest, the splits slowest
+  b = xcd_run(b, tiles_wgs);
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int tile = b % tiles, split = b / tiles;
+  const int nk_all = (int)(p.K / kBK);
+  const int kt0 = (int)((int64_t)nk_all * split / p.splits);
+  const int nk = (int)((int64_t)nk_all * (split + 1) / p.splits) - kt0;
+  float* part = p.splits > 1 ? p.part + ((int64_t)tile * p.splits + split) * kMidRows * kTile : nullptr;
+  gemm_tile<TRANS, EPI, kMidRows, kTile, 2, kMidStages, false>(
+      p, (int64_t)(tile % p.tiles_m) * kMidRows, (int64_t)(tile / p.tiles_m) * kTile, kt0, nk, part,
+      S, S + kMidStages * kMidRows * kBK, nullptr);
+}
+
+// Split-K, second launch: one wave per 32 x 32 block of a tile of BM x 256 sums the block's split
+// partials in split order (fixed, so the result is deterministic) and runs the epilogue on it.
+// The kernel boundary orders it after every partial store.
+template <bool TRANS, int EPI, int BM>
 __global__ __launch_bounds__(64) void hgemm_reduce_kernel(GemmParams p) {
   // 8 KB of LDS per one-wave workgroup, so that 20 of them fit a CU
   __shared__ __attribute__((aligned(16))) uint8_t escr[epi_scratch_bytes(1)];
-  constexpr int TM = 4, TN = 2;   // the blocks of one 128 x 64 wave block of the first launch
+  constexpr int TM = BM / 64, TN = 2;   // the blocks of one (BM / 2) x 64 wave block of the first launch
+  constexpr int BLOCKS = 8 * TM * TN;
   const int lane = threadIdx.x;
-  const int tile = blockIdx.x / 64, blk = blockIdx.x % 64;
+  const int tile = blockIdx.x / BLOCKS, blk = blockIdx.x % BLOCKS;
   const int wave = blk / (TM * TN), i = (blk / TN) % TM, j = blk % TN;
-  const int64_t m0 = (int64_t)(tile % p.tiles_m) * kTile + (wave / 4) * 128 + 32 * i;
+  const int64_t m0 = (int64_t)(tile % p.tiles_m) * BM + (wave / 4) * (BM / 2) + 32 * i;
   const int64_t n0 = (int64_t)(tile / p.tiles_m) * kTile + (wave % 4) * 64 + 32 * j;
   if (m0 >= p.M) return;
-  const float* src = p.part + (int64_t)tile * p.splits * kTile * kTile +
+  const float* src = p.part + (int64_t)tile * p.splits * BM * kTile +
                      (wave * TM * TN + i * TN + j) * 1024 + 4 * lane;
   f32x16 acc[1][1];
   f32x4 v_all[4][4];
@@ -1036,7 +1086,7 @@ __global__ __launch_bounds__(64) void hgemm_reduce_kernel(GemmParams p) {
       const int s = sp + u < p.splits ? sp + u : p.splits - 1;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        v_all[u][q] = *reinterpret_cast<const f32x4*>(src + (int64_t)s * kTile * kTile + 256 * q);
+        v_all[u][q] = *reinterpret_cast<const f32x4*>(src + (int64_t)s * BM * kTile + 256 * q);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -1063,6 +1113,7 @@ int cu_count() {
 // The launch shape of a GEMM on this kernel, or ok = false.
 struct HPlan {
   bool ok;
+  bool mid;     // 128 x 256 tiles (hgemm_mid_kernel): main_wgs of them, splits included
   int64_t tiles_m, tiles_n, main_wgs, tail_wgs;
   int splits;
   int xcd_gm;   // GemmParams::xcd_gm
@@ -1090,67 +1141,139 @@ int xcd_blocks(int64_t tiles_m, int64_t main_wgs, int64_t tail_wgs, int qbase) {
   return best;
 }
 
-HPlan hplan_tiles(int64_t M, int64_t N, int64_t K, int epi, bool no_split, bool nt) {
-  HPlan h{false, 0, 0, 0, 0, 1, 0};
-  if (M <= 0 || N % kTile || K % kBK || K < kBK) return h;
-  const int cus = cu_count();
-  if (cus <= 0) return h;
-  h.tiles_m = (M + kTile - 1) / kTile;
-  h.tiles_n = N / kTile;
-  const int64_t tiles = h.tiles_m * h.tiles_n;
-  if (tiles * 4 > 0x7fffffff) return h;
-  if (tiles >= cus) {
-    // a last round at most half full runs as 128 x 128 quarters
-    h.main_wgs = tiles;
-    const int64_t rest = tiles % cus;
-    if (rest > 0 && rest <= cus / 2) {
-      h.main_wgs = tiles - rest;
-      h.tail_wgs = 4 * rest;
-    }
-    h.ok = true;
-    return h;
+// At least one 256 x 256 tile per CU: rounds of them, a last round at most half full as 128 x 128
+// quarters.
+HPlan hplan_rounds(int64_t M, int64_t N, int cus) {
+  HPlan h{true, false, (M + kTile - 1) / kTile, N / kTile, 0, 0, 1, 0};
+  const int64_t tiles = h.tiles_m * h.tiles_n, rest = tiles % cus;
+  h.main_wgs = tiles;
+  if (rest > 0 && rest <= cus / 2) {
+    h.main_wgs = tiles - rest;
+    h.tail_wgs = 4 * rest;
   }
-  // fewer tiles than CUs: split K so that the splits fill the CUs once.  The fp32 partials cost
-  // two passes over splits x tiles x 256 KB, which only long K (4096 or more) repays; LINEAR
-  // only, at least 4 row tiles.  NT GEMMs whose 128 x 128 quarters fill half the CUs run as
-  // quarters over the whole K instead: their loop (computing and loading waves apart) does as
-  // much per CU as the full tiles' in the step, without the partials' round trip or the reduce
-  // launch (down forward at M = 2048, K = 8960: 71.8 -> 61.8 us in the step)
-  const int64_t quarters = (M + 127) / 128 * (N / 128);
-  if (!no_split && epi == EPI_LINEAR && h.tiles_m >= 4 && K >= 4096 &&
-      !(nt && quarters * 2 >= cus)) {
-    int64_t s = cus / tiles;
-    if (s > K / kBK / 8) s = K / kBK / 8;
-    if (s >= 2) {
-      h.splits = (int)s;
-      h.main_wgs = tiles * s;
-      h.ok = true;
-      return h;
-    }
-  }
-  // otherwise every tile as 128 x 128 quarters, when they fill at least half the CUs
-  if (quarters * 2 < cus && !no_split) return h;
-  h.main_wgs = 0;
-  h.tail_wgs = 4 * tiles;
-  h.ok = true;
   return h;
 }
 
-HPlan hplan(int64_t M, int64_t N, int64_t K, int epi, bool no_split, bool nt) {
-  HPlan h = hplan_tiles(M, N, K, epi, no_split, nt);
-  if (h.ok && h.splits == 1)
+// Estimated microseconds of the plans for fewer tiles than CUs.  A round of workgroups takes
+// fixed + steps (step + load * busy), busy the share of the CUs it fills (the clock, the LDS-DMA
+// loads and the L2s are shared); split K adds its partials' round trip.  The constants are fits to
+// every plan at 20 (operation, N, K) and 26 row counts from 64 to 8192 on MI355X (graph replays;
+// the fits are within 5 % in the mean), and the plan of least estimated time was within 8 % of
+// the fastest at every one of those sizes.  Against the rules they replace (128 x 128 tiles where
+// they fill half the CUs, split 256 x 256 tiles from four row tiles on, w4gemm.hip's kernel
+// elsewhere) the plans gain 11 % in the mean: o forward at M = 1024 22.9 -> 16.0 us, down forward
+// at M = 701 52 -> 34 and M = 3000 120 -> 85, down^T backward at M = 853 54 -> 36 and M = 1400
+// 72 -> 51, gate|up forward at M = 701 54 -> 41, gate|up dX at M = 701 91 -> 55.
+struct PlanCost {
+  float fixed, step, load;
+  float reduce, tbps;   // split K: the reduce launch, TB/s of the partials' bytes
+};
+enum { COST_QUARTERS, COST_MID, COST_FULL, COST_STAGED128, COST_STAGED64, COST_KINDS };
+constexpr PlanCost kCost[4][COST_KINDS] = {
+    // LINEAR NT
+    {{6.8f, 0.325f, 0.08f, 0, 1}, {8.6f, 0.66f, 0.11f, 2.5f, 3.8f}, {12.9f, 1.015f, 0.275f, 0, 4.6f},
+     {0.0f, 0.38f, 1.0f, 7.1f, 2.7f}, {1.5f, 0.137f, 0.244f, 6.7f, 2.1f}},
+    // LINEAR NN
+    {{5.6f, 0.467f, 0.054f, 0, 1}, {7.5f, 0.79f, 0.076f, 2.8f, 3.4f}, {10.3f, 1.07f, 0.30f, 0, 3.9f},
+     {11.9f, 0.02f, 1.63f, 2.6f, 50.0f}, {8.1f, 0.0f, 1.03f, 1.6f, 27.0f}},
+    // SWIGLU_FWD
+    {{6.8f, 0.28f, 0.073f, 0, 1}, {7.8f, 0.64f, 0.11f, 0, 1}, {12.2f, 0.825f, 0.43f, 0, 1},
+     {4.8f, 0.57f, 0.31f, 0, 1}, {0, 1e6f, 0, 0, 1}},
+    // SWIGLU_BWD
+    {{9.6f, 0.325f, 0.116f, 0, 1}, {14.2f, 0.514f, 0.343f, 0, 1}, {22.5f, 0.6f, 0.76f, 0, 1},
+     {11.2f, 0.65f, 1.69f, 0, 1}, {11.2f, 0.65f, 1.69f, 0, 1}},
+};
+
+// `wgs` workgroups on `slots` places at once, `steps` K steps each, `bytes` of fp32 partials
+float plan_us(const PlanCost& c, int64_t wgs, int64_t slots, float steps, int64_t bytes) {
+  const int64_t full = wgs / slots, rest = wgs % slots;
+  float t = full * (c.fixed + steps * (c.step + c.load));
+  if (rest) t += c.fixed + steps * (c.step + c.load * (float)rest / (float)slots);
+  return bytes ? t + c.reduce + (float)bytes / (c.tbps * 1e6f) : t;
+}
+
+// 128 x 256 tiles over `splits` ranges of K.
+HPlan hplan_mid(int64_t M, int64_t N, int splits) {
+  HPlan h{true, true, 0, 0, 0, 0, splits, 0};
+  h.tiles_m = (M + kMidRows - 1) / kMidRows;
+  h.tiles_n = N / kTile;
+  h.main_wgs = h.tiles_m * h.tiles_n * splits;
+  return h;
+}
+
+// The plan for fewer 256 x 256 tiles than CUs: the cheapest by the estimate above; ok = false when
+// that is w4gemm.hip's kernel (never for rope: the rotary epilogue runs here only).  split: the
+// caller has room for the partials (the rotary epilogue pairs the two column halves of a head
+// inside one workgroup, so it takes no split K either).
+HPlan hplan_small(int64_t M, int64_t N, int64_t K, int epi, bool split, bool rope, bool nt, int cus) {
+  const PlanCost* cost = kCost[epi == EPI_LINEAR ? (nt ? 0 : 1) : epi == EPI_SWIGLU_FWD ? 2 : 3];
+  const int64_t tm = (M + kTile - 1) / kTile, tn = N / kTile;
+  const int64_t tm2 = (M + kMidRows - 1) / kMidRows;
+  const float nk = (float)(K / kBK);
+  const int max_splits = epi == EPI_LINEAR && split && !rope ? (int)(K / kBK / 4) : 1;
+  HPlan best{true, false, tm, tn, 0, 4 * tm * tn, 1, 0};   // every tile as 128 x 128 quarters
+  float t_best = plan_us(cost[COST_QUARTERS], tm2 * (N / 128), cus, nk, 0);
+  auto consider = [&](float t, const HPlan& h) {
+    if (t < t_best) {
+      t_best = t;
+      best = h;
+    }
+  };
+  for (int s = 1; s == 1 || (s <= max_splits && tm * tn * s <= cus); ++s)
+    consider(plan_us(cost[COST_FULL], tm * tn * s, cus, nk / s,
+                     s > 1 ? tm * tn * s * kTile * kTile * 4 : 0),
+             HPlan{true, false, tm, tn, tm * tn * s, 0, s, 0});
+  for (int s = 1; s == 1 || (s <= max_splits && tm2 * tn * s <= cus); ++s)
+    consider(plan_us(cost[COST_MID], tm2 * tn * s, cus, nk / s,
+                     s > 1 ? tm2 * tn * s * kMidRows * kTile * 4 : 0),
+             hplan_mid(M, N, s));
+  if (!rope) {
+    Plan st = plan_for(M, N, K, epi);
+    if (!split) st.splits = 1;
+    if (plan_us(cost[st.bn == 128 ? COST_STAGED128 : COST_STAGED64], st.tiles * st.splits, 2 * cus,
+                nk / st.splits, st.splits > 1 ? st.tiles * st.splits * st.bm * st.bn * 4 : 0) <= t_best)
+      best.ok = false;
+  }
+  return best;
+}
+
+// w4: the plan of the NF4-reading form, which has no 128 x 256 tiles: where the fp16 form runs them
+// it takes 128 x 128 tiles (the same sums) or, with split K (other sums), declines.
+HPlan hplan(int64_t M, int64_t N, int64_t K, int epi, bool split, bool rope, bool nt, bool w4) {
+  HPlan h{false, false, 0, 0, 0, 0, 1, 0};
+  if (M <= 0 || N % kTile || K % kBK || K < kBK) return h;
+  const int cus = cu_count();
+  if (cus <= 0) return h;
+  const int64_t tiles = (M + kTile - 1) / kTile * (N / kTile);
+  if (tiles * 4 > 0x7fffffff) return h;
+  h = tiles >= cus ? hplan_rounds(M, N, cus) : hplan_small(M, N, K, epi, split, rope, nt, cus);
+  if (w4 && h.ok && h.mid) {
+    if (h.splits > 1) return HPlan{false, false, 0, 0, 0, 0, 1, 0};
+    h = HPlan{true, false, (M + kTile - 1) / kTile, N / kTile, 0, 4 * tiles, 1, 0};
+  }
+  if (h.ok && !h.mid && h.splits == 1)
     h.xcd_gm = xcd_blocks(h.tiles_m, h.main_wgs, h.tail_wgs,
                           epi == EPI_SWIGLU_BWD ? 0 : (int)h.main_wgs);
   return h;
 }
 
+int64_t partial_bytes(const HPlan& h) {
+  return h.splits > 1 ? h.main_wgs * (h.mid ? kMidRows : kTile) * kTile * (int64_t)sizeof(float) : 0;
+}
+
 }  // namespace
 
+// Partials of the plan, or of the 256 x 256 tiles' own split over every CU where that is more (a
+// caller's buffer then holds either).
 int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
-  const HPlan h = hplan(M, N, K, epi, false, nt);
+  const HPlan h = hplan(M, N, K, epi, true, false, nt, false);
   if (!h.ok) return -1;
   if (h.splits == 1) return 0;
-  return h.main_wgs * kTile * kTile * (int64_t)sizeof(float);
+  const int64_t tiles = (M + kTile - 1) / kTile * (N / kTile);
+  int64_t s = cu_count() / tiles;
+  if (s > K / kBK / 8) s = K / kBK / 8;
+  const int64_t own = partial_bytes(h), full = tiles * s * kTile * kTile * (int64_t)sizeof(float);
+  return own > full ? own : full;
 }
 
 // The epilogue writes 16-byte vectors of 8 consecutive columns.
@@ -1170,8 +1293,6 @@ int hgemm_launch(const GemmParams& p0, void* ws, int64_t ws_bytes, hipStream_t s
            : p0.w16 != nullptr) ||
       !vector_outputs_ok(p0, EPI))
     return kHgemmDeclined;
-  // the rotary epilogue pairs the two column halves of a head inside one workgroup: no split-K,
-  // and 128-column tiles at any size
   const bool rope = p0.rope_pos != nullptr;
   if (rope && (TRANS || EPI != EPI_LINEAR)) return kHgemmDeclined;
   // the loads' 32-bit byte offsets: A within a 256-row tile, W (NT) within the whole weight
@@ -1180,19 +1301,17 @@ int hgemm_launch(const GemmParams& p0, void* ws, int64_t ws_bytes, hipStream_t s
   if ((kTile * p0.lda + p0.K) * (int64_t)sizeof(f16) >= kOffMax ||
       (!W4 && (TRANS ? (int64_t)kBK * p0.N : p0.N * p0.K) * (int64_t)sizeof(f16) >= kOffMax))
     return kHgemmDeclined;
-  const HPlan h = hplan(p0.M, p0.N, p0.K, EPI, rope, !TRANS);
+  HPlan h = hplan(p0.M, p0.N, p0.K, EPI, true, rope, !TRANS, W4);
+  // split K without room for its partials: the best plan without
+  if (h.ok && partial_bytes(h) > 0 && (!ws || ws_bytes < partial_bytes(h) || !dk_aligned(ws, 256)))
+    h = hplan(p0.M, p0.N, p0.K, EPI, false, rope, !TRANS, W4);
   if (!h.ok) return kHgemmDeclined;
   GemmParams p = p0;
   p.tiles_m = (int)h.tiles_m;
   p.tiles_n = (int)h.tiles_n;
   p.splits = h.splits;
   p.xcd_gm = h.xcd_gm;
-  if (h.splits > 1) {
-    // the partials go to the caller's workspace; without room for them, decline
-    if (!ws || ws_bytes < h.main_wgs * kTile * kTile * (int64_t)sizeof(float) || !dk_aligned(ws, 256))
-      return kHgemmDeclined;
-    p.part = reinterpret_cast<float*>(ws);
-  }
+  if (h.splits > 1) p.part = reinterpret_cast<float*>(ws);
   // carried dequant: the given workgroup count, or (auto) the CUs the last round leaves idle
   int side = 0;
   if (p.side.sb1 > p.side.sb0 && p.side.wgs != 0) {
@@ -1207,6 +1326,21 @@ int hgemm_launch(const GemmParams& p0, void* ws, int64_t ws_bytes, hipStream_t s
   // carried LoRA column sums (NN LINEAR only; the caller sets p.sums.wgs)
   const int sums = TRANS && EPI == EPI_LINEAR ? p.sums.wgs : 0;
   p.sums.wgs = sums;
+  if constexpr (!W4) {
+    if (h.mid) {
+      hipLaunchKernelGGL((hgemm_mid_kernel<TRANS, EPI>), dim3((unsigned)(h.main_wgs + sums + side)),
+                         dim3(kThreads), 0, stream, p, (int)h.main_wgs);
+      DK_CHECK_LAUNCH();
+      if constexpr (EPI == EPI_LINEAR) {
+        if (h.splits > 1) {
+          hipLaunchKernelGGL((hgemm_reduce_kernel<TRANS, EPI, kMidRows>),
+                             dim3((unsigned)(h.tiles_m * h.tiles_n * 32)), dim3(64), 0, stream, p);
+          DK_CHECK_LAUNCH();
+        }
+      }
+      return 0;
+    }
+  }
   // the fp16 SwiGLU GEMMs that take more than one round run one persistent workgroup per CU
   // when their tiles divide evenly over the XCDs' CUs
   const int cus = cu_count();
@@ -1221,7 +1355,7 @@ int hgemm_launch(const GemmParams& p0, void* ws, int64_t ws_bytes, hipStream_t s
   DK_CHECK_LAUNCH();
   if constexpr (EPI == EPI_LINEAR) {   // hplan splits K for the LINEAR epilogue only
     if (h.splits > 1) {
-      hipLaunchKernelGGL((hgemm_reduce_kernel<TRANS, EPI>),
+      hipLaunchKernelGGL((hgemm_reduce_kernel<TRANS, EPI, kTile>),
                          dim3((unsigned)(h.tiles_m * h.tiles_n * 64)), dim3(64), 0, stream, p);
       DK_CHECK_LAUNCH();
     }

@@ -38,7 +38,6 @@ using namespace dk;
 
 namespace {
 
-constexpr int kBK = 64;
 constexpr int kStride = kBK + 8;  // halves per K-contiguous LDS row (144 bytes)
 constexpr int kPadT = 16;         // NN: halves of padding per N-contiguous LDS row of the W tile
 // Waves per role: consumers are WAVES_M x 2 (64-row strips), producers as many; 128-row tiles
@@ -571,33 +570,6 @@ void w4_gemm_kernel(GemmParams p) {
   }
 }
 
-// Launch plan: tile shape and split-K factor.  256 CUs.  A 128-row tile's workgroup needs
-// 76.8 KB of LDS (60 KB at 64 columns) and at most 128 VGPRs, so two share a CU (512 slots).
-// (256 x 128 tiles, one workgroup per CU, measured slower at these shapes and are not
-// planned.)  Shapes with fewer tiles than slots split K (at least 8 steps per split) so that about
-// 768 workgroups run: the fp32 partial tiles cost one extra pass over the output in the second
-// launch, so short K (under 64 steps) prefers narrower tiles and splits only below 256 tiles.
-struct Plan {
-  int bm, bn, splits;
-  int64_t tiles;
-};
-
-Plan plan_for(int64_t M, int64_t N, int64_t K, int epi) {
-  const int64_t nk = K / kBK;
-  const int64_t mt128 = (M + 127) / 128;
-  Plan pl{128, 128, 1, mt128 * (N / 128)};
-  if (N % 128 != 0) pl = {128, 64, 1, mt128 * (N / 64)};
-  if (epi != EPI_LINEAR || pl.tiles >= 512) return pl;
-  if (pl.bn == 128 && nk < 64) pl = {128, 64, 1, mt128 * (N / 64)};
-  if ((pl.tiles < 256 && nk >= 16) || (pl.tiles < 512 && nk >= 64)) {
-    int64_t s = (768 + pl.tiles - 1) / pl.tiles;
-    if (s > nk / 8) s = nk / 8;
-    if (s > 8) s = 8;
-    if (s >= 2) pl.splits = (int)s;
-  }
-  return pl;
-}
-
 // Two-phase path: with many row tiles, dequantising each W tile once per row tile (in LDS) costs
 // more LDS bandwidth than the MFMAs can hide, so from kTwoPhaseRows rows and kTwoPhaseCols
 // output columns on, the weight is first dequantised once into the workspace at HBM rate
@@ -609,7 +581,13 @@ Plan plan_for(int64_t M, int64_t N, int64_t K, int epi) {
 constexpr int64_t kTwoPhaseRows = 512;
 constexpr int64_t kTwoPhaseCols = 1536;
 
-bool two_phase(int64_t M, int64_t N) { return M >= kTwoPhaseRows && N >= kTwoPhaseCols; }
+//
+// Narrower outputs join them where the fp16 GEMM splits K.  (The 256-tile kernel can dequantise
+// the W tiles itself, bit-identically, but its per-step conversion costs more than the dequant
+// launch: gate|up dX at M = 853 82 + 10 us against 17 + 59 + 7.)
+bool two_phase(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
+  return M >= kTwoPhaseRows && (N >= kTwoPhaseCols || hgemm_workspace(M, N, K, epi, nt) > 0);
+}
 
 int64_t round256(int64_t b) { return (b + 255) / 256 * 256; }
 
@@ -618,17 +596,18 @@ int64_t plan_workspace(const Plan& pl) {
   return pl.tiles * pl.splits * pl.bm * pl.bn * (int64_t)sizeof(float);
 }
 
-// Workspace of one GEMM: [split-K partial tiles | fp16 weight (two-phase)].
-// Workspace of an NF4-reading GEMM: room for whichever path dispatch takes, the 256-tile kernel's
-// split-K partials (reading NF4 itself), or the 128 x 128 kernel's partials with the fp16 weight
-// after them (two-phase shapes).
+// Bytes of split-K partials of an NF4-reading GEMM: room for whichever kernel dispatch runs.
+int64_t partials(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
+  const int64_t own = plan_workspace(plan_for(M, N, K, epi));
+  const int64_t tile = hgemm_workspace(M, N, K, epi, nt);
+  return round256(own > tile ? own : tile);
+}
+
+// Workspace of an NF4-reading GEMM: [split-K partial tiles | fp16 weight (two-phase)].
 int64_t gemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
   if (M <= 0) return 0;
-  const int64_t part = plan_workspace(plan_for(M, N, K, epi));
-  const int64_t w16 = two_phase(M, N) ? N * K * (int64_t)sizeof(f16) : 0;
-  const int64_t own = w16 ? round256(part) + w16 : part;
-  const int64_t tile = hgemm_workspace(M, N, K, epi, nt);
-  return own > tile ? own : tile;
+  const int64_t w16 = two_phase(M, N, K, epi, nt) ? N * K * (int64_t)sizeof(f16) : 0;
+  return partials(M, N, K, epi, nt) + w16;
 }
 
 template <int BM, int BN, bool TRANS, int EPI, bool F16B>
@@ -670,19 +649,13 @@ int launch_plan(const Plan& pl, GemmParams p, hipStream_t stream) {
 // Runs the plan.  Without a workspace: one phase (W dequantised in LDS), no split-K.  With one
 // (at least gemm_workspace bytes): split-K partials and, on the two-phase shapes, the weight
 // dequantised to fp16 in the workspace first (both launches on `stream`, in order).  The weight's
-// `kernel` field picks the 256-tile kernel reading NF4: where it is fastest (AUTO: split-K
-// plans), wherever its plan takes the shape (TILE), or never (STAGED).
+// `kernel` field asks for the 256-tile kernel reading NF4 wherever its plan takes the shape (TILE).
 
 template <bool TRANS, int EPI>
 int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, hipStream_t stream) {
   if (ws && ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
-  // the 256-tile kernel with the weight dequantised in LDS (W4) where its plan splits K (few
-  // output tiles, long K): there it beats the separate dequant + fp16 GEMM (gate|up dX at
-  // M = 2048: 179 against 188 us); elsewhere its per-step conversion costs more than the
-  // dequant launch saves (measured on every config-4 shape), and the paths below run
-  const int mode = w->kernel;
-  if (mode == DK_W4_KERNEL_TILE ||
-      (mode == DK_W4_KERNEL_AUTO && ws && hgemm_workspace(p.M, p.N, p.K, EPI, !TRANS) > 0)) {
+  // the 256-tile kernel with the weight dequantised in LDS, on request only (see two_phase)
+  if (w->kernel == DK_W4_KERNEL_TILE) {
     const int r = hgemm_launch<TRANS, EPI, true>(p, ws, ws_bytes, stream);
     if (r != kHgemmDeclined) return r;
   }
@@ -691,16 +664,16 @@ int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, h
     pl.splits = 1;
     return launch_plan<TRANS, EPI, false>(pl, p, stream);
   }
-  if (ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
   if (!dk_aligned(ws, 256)) return DK_ERR_ALIGN;
   if (pl.splits > 1) p.part = reinterpret_cast<float*>(ws);
-  if (!two_phase(p.M, p.N)) return launch_plan<TRANS, EPI, false>(pl, p, stream);
-  f16* w16 = reinterpret_cast<f16*>(reinterpret_cast<char*>(ws) + round256(plan_workspace(pl)));
+  if (!two_phase(p.M, p.N, p.K, EPI, !TRANS)) return launch_plan<TRANS, EPI, false>(pl, p, stream);
+  const int64_t part_bytes = partials(p.M, p.N, p.K, EPI, !TRANS);
+  f16* w16 = reinterpret_cast<f16*>(reinterpret_cast<char*>(ws) + part_bytes);
   if (int e = dk_nf4_dequant(w->packed, w->qabs, w->scale2, w->offset2, w->code2, w->nf4, w16,
                              w->rows * w->cols / DK_QBLOCK, stream))
     return e;
   p.w16 = w16;
-  const int big = hgemm_launch<TRANS, EPI>(p, nullptr, 0, stream);
+  const int big = hgemm_launch<TRANS, EPI>(p, ws, part_bytes, stream);
   if (big != kHgemmDeclined) return big;
   return launch_plan<TRANS, EPI, true>(pl, p, stream);
 }

@@ -50,8 +50,8 @@ typedef struct dk_nf4_weight {
  * workspace).  The 256 x 256-tile kernel can read the packed NF4 weight itself, each workgroup
  * dequantising its W tiles into LDS (bit-identical to the fp16-weight form); otherwise the weight
  * is first dequantised into the workspace and read as fp16, or the 128 x 128 warp-specialised
- * kernel dequantises in LDS.  AUTO: the tile kernel reads NF4 where that is fastest (its split-K
- * plans: few output tiles, long K); TILE: wherever its plan takes the shape; STAGED: never.  The
+ * kernel dequantises in LDS.  TILE: the tile kernel reads NF4 wherever its plan takes the shape;
+ * STAGED: never; AUTO: the library's choice (as STAGED: the dequant launch measures faster).  The
  * choice travels with each call's weight argument: the library keeps no setting of its own. */
 #define DK_W4_KERNEL_AUTO 0
 #define DK_W4_KERNEL_TILE 1
@@ -235,7 +235,8 @@ int dk_w4_linear_fwd_lora(const void* x, int64_t ldx, int64_t m, const dk_nf4_we
 
 /* Workspace of the fused NF4 GEMMs.  No counterpart in the reference (cuBLAS manages its own);
  * it stands in for the reference's fp16 dequant workspace (solution/fast_qwen.py:398-418).
- * It holds split-K partial tiles and, from 512 rows on for outputs of at least 1536 columns, the
+ * It holds split-K partial tiles and, from 512 rows on for outputs of at least 1536 columns (and
+ * narrower ones whose fp16 GEMM splits K), the
  * weight dequantised to fp16 once per call (the "two-phase" path: dequant at HBM rate, then the
  * MFMA GEMM on fp16 W), which at many row tiles is faster than dequantising each W tile again for
  * every row tile.  Without a
