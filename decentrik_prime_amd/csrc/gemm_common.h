@@ -96,6 +96,13 @@ constexpr int kHgemmDeclined = -1000;
 // p.w16) and dequantised by each workgroup into LDS, bit-identical to the fp16 form's results.
 template <bool TRANS, int EPI, bool W4 = false>
 int hgemm_launch(const GemmParams& p, void* ws, int64_t ws_bytes, hipStream_t stream);
+// The NT GEMM of `p` for a few rows (skinny.hip), on packed NF4 weights or p.w16: up to 16 rows, or
+// 32 for a LINEAR weight of at most 2048 x 1536.
+inline bool skinny_takes(const GemmParams& p, int epi) {
+  return p.M <= 16 || (p.M <= 32 && epi == EPI_LINEAR && p.N * p.K <= (int64_t)2048 * 1536);
+}
+template <int EPI, bool F16>
+int skinny_launch(const GemmParams& p, hipStream_t stream);
 // Split-K partials the launch of that shape needs (0: no split; -1: the plan does not take the
 // shape); nt: NT (W stored [N][K]).
 int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt);

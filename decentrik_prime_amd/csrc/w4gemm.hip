@@ -654,6 +654,10 @@ int launch_plan(const Plan& pl, GemmParams p, hipStream_t stream) {
 template <bool TRANS, int EPI>
 int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, hipStream_t stream) {
   if (ws && ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
+  // a few rows: every weight converted once, one launch, no workspace
+  if constexpr (!TRANS) {
+    if (skinny_takes(p, EPI)) return skinny_launch<EPI, false>(p, stream);
+  }
   // the 256-tile kernel with the weight dequantised in LDS, on request only (see two_phase)
   if (w->kernel == DK_W4_KERNEL_TILE) {
     const int r = hgemm_launch<TRANS, EPI, true>(p, ws, ws_bytes, stream);
@@ -880,6 +884,12 @@ int dispatch_h16(GemmParams p, const void* w16, void* ws, int64_t ws_bytes,
     p.sums.jobs = sums.jobs;
     p.sums.rows = sums.rows;
     p.sums.wgs = sums.blocks;
+  }
+  if constexpr (!TRANS) {
+    if (skinny_takes(p, EPI)) {   // no tiles to carry other work (NT GEMMs have no column sums)
+      if (int e = skinny_launch<EPI, true>(p, stream)) return e;
+      return side_alone(p.side, stream);
+    }
   }
   const int big = hgemm_launch<TRANS, EPI>(p, ws, ws_bytes, stream);
   if (big != kHgemmDeclined) return big ? big : (carry ? 0 : sums_alone());
