@@ -184,9 +184,21 @@ def check(rc, what):
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = None
 
 
 def stream_handle(device=None):
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream of `device` as the integer handle the C ABI takes (0: the default
+    stream), without building a torch.cuda.Stream object per call."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        _raw_stream = torch._C._cuda_getCurrentRawStream
+    index = device.index if device is not None else None
+    if index is None:
+        import torch
+        index = torch.cuda.current_device()
+    return _raw_stream(index)

@@ -94,6 +94,18 @@ def nf4_table(device):
     return torch.tensor(NF4_CODE, dtype=torch.float32, device=device)
 
 
+_NF4 = {}
+
+
+def nf4_on(device):
+    """nf4_table, one tensor per device (a new table is a copy from the host that waits)."""
+    device = torch.device(device)
+    t = _NF4.get(device)
+    if t is None:
+        t = _NF4[device] = nf4_table(device)
+    return t
+
+
 def quantize_into(w16, code2, nf4, packed, qabs, scale2, offset2):
     """Quantise the fp16 CUDA tensor ``w16`` into caller-provided section views (the four sections
     of a repacked layer, or standalone tensors)."""
@@ -119,7 +131,7 @@ def quantize_4bit(w16, code2=None):
     """NF4 + double quantisation of an fp16 CUDA weight [rows, cols] -> Params4bit."""
     dev = w16.device
     code2 = code2_on(dev) if code2 is None else code2
-    nf4 = nf4_table(dev)
+    nf4 = nf4_on(dev)
     n = w16.numel()
     packed = torch.empty(n // 2, dtype=torch.uint8, device=dev)
     qabs = torch.empty(n // 64, dtype=torch.uint8, device=dev)

@@ -15,7 +15,7 @@ import threading
 import torch
 
 from . import _lib
-from .quant import code2_on, nf4_table
+from .quant import code2_on, nf4_on, nf4_table
 
 
 class W4:
@@ -43,6 +43,7 @@ class W4:
         self._c = _lib.NF4WeightC(packed.data_ptr(), qabs.data_ptr(), scale2.data_ptr(),
                                   offset2.data_ptr(), code2.data_ptr(), nf4.data_ptr(),
                                   self.rows, self.cols, self.kernel)
+        self._ref = ctypes.byref(self._c)
 
     def with_kernel(self, kernel):
         """The same weight (the same section tensors) with another ``kernel`` choice."""
@@ -58,8 +59,7 @@ class W4:
         return self.packed.device
 
     def c_ref(self):
-        import ctypes
-        return ctypes.byref(self._c)
+        return self._ref
 
     @classmethod
     def from_sections(cls, packed, qabs, scale2, offset2, start, rows, cols, code2, nf4):
@@ -80,7 +80,7 @@ class W4:
         offset2 = qs.offset.float().reshape(1).expand(n // 16384).contiguous().to(dev)
         return cls(param.data.reshape(-1), qs.absmax.reshape(-1), qs.state2.absmax.reshape(-1).float(),
                    offset2, qs.state2.code.float().to(dev),
-                   nf4 if nf4 is not None else nf4_table(dev), rows, cols)
+                   nf4 if nf4 is not None else nf4_on(dev), rows, cols)
 
     def dequantize(self, out=None):
         """fp16 [rows, cols] (the reference's workspace view of this weight)."""
@@ -94,34 +94,45 @@ class W4:
 
 _WS = {}
 _WS_LOCK = threading.Lock()
+_BYTES = {}     # (form, m, rows, cols, op, device index) -> workspace bytes
+_BYTES_MOST = 4096
+
+
+def _scratch(nbytes, device):
+    """Scratch of the fused GEMMs on the current stream: one buffer per (device, stream), grown on
+    demand.  Kernels on one stream run in order, so they share it."""
+    key = (device, _lib.stream_handle(device))
+    with _WS_LOCK:
+        buf = _WS.get(key)
+        if buf is None or buf.numel() < nbytes:
+            buf = _WS[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    return buf
+
+
+def _needed(key, query):
+    """Workspace bytes of one shape: a function of the sizes and the device's CU count alone, so
+    each is asked of the library once."""
+    nbytes = _BYTES.get(key)
+    if nbytes is None:
+        if len(_BYTES) >= _BYTES_MOST:
+            _BYTES.clear()
+        nbytes = _BYTES[key] = int(query())
+    return nbytes
 
 
 def _workspace(w, m, op, device):
     """Scratch of a fused NF4 GEMM (split-K partials and the two-phase fp16 weight; None when the
-    shape needs none): one buffer per (device, stream), grown on demand.  Kernels on one stream
-    run in order, so they share it."""
-    nbytes = int(_lib.lib().dk_w4_workspace(m, w.c_ref(), int(op)))
-    if nbytes == 0:
-        return None, 0
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
-    with _WS_LOCK:
-        buf = _WS.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = _WS[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    return buf, nbytes
+    shape needs none)."""
+    nbytes = _needed((4, m, w.rows, w.cols, op, device.index),
+                     lambda: _lib.lib().dk_w4_workspace(m, w.c_ref(), int(op)))
+    return (_scratch(nbytes, device), nbytes) if nbytes else (None, 0)
 
 
 def _h16_workspace(m, rows, cols, op, device):
     """Split-K scratch of an fp16-weight GEMM (None when the shape needs none)."""
-    nbytes = int(_lib.lib().dk_h16_workspace(m, rows, cols, int(op)))
-    if nbytes == 0:
-        return None, 0
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
-    with _WS_LOCK:
-        buf = _WS.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = _WS[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    return buf, nbytes
+    nbytes = _needed((16, m, rows, cols, op, device.index),
+                     lambda: _lib.lib().dk_h16_workspace(m, rows, cols, int(op)))
+    return (_scratch(nbytes, device), nbytes) if nbytes else (None, 0)
 
 
 def _check_w16(w16, w):
@@ -651,8 +662,9 @@ class QLoRALinearFunction(torch.autograd.Function):
         mask = mask if ctx.has_mask else None
         dy = dy.contiguous().half()
         da, db, dz = lora_grads(dy, z, x, b16, ctx.s, mask, ctx.ks)
-        dx = linear_backward_dx(dy, ctx.w, dz, a16, mask, ctx.ks, out_dtype=torch.float32)
-        return (dx.to(x.dtype), da.to(ctx.dtypes[0]), db.to(ctx.dtypes[1]),
+        # in x's own dtype: the GEMM's one rounding of the fp32 sum, no fp32 copy of dx
+        dx = linear_backward_dx(dy, ctx.w, dz, a16, mask, ctx.ks, out_dtype=x.dtype)
+        return (dx, da.to(ctx.dtypes[0]), db.to(ctx.dtypes[1]),
                 None, None, None, None, None)
 
 
