@@ -160,3 +160,41 @@ def test_repacked_layer_dequant_and_split(torch_dev):
     k_nf4.dequant_range(packed, 0, split, code2, nf4t, out3)
     torch.cuda.synchronize()
     assert torch.equal(out3, out)
+
+
+def test_quantiser_other_tables(torch_dev):
+    """Code tables whose midpoints the bucket search cannot take (two in one bucket, outside the
+    range) fall back to the plain count; a table with a midpoint on a bucket's edge (0.25) and
+    weights one fp16 step around every midpoint do not: codes equal to counting the midpoints
+    below w * fp32(1 / absmax)."""
+    torch = torch_dev
+    from decentrik_prime_amd import quant
+    code2 = quant.code2_on("cuda")
+    usual = torch.tensor(quant.NF4_CODE, dtype=torch.float32)
+    edge = usual.clone()
+    edge[10], edge[11] = 0.24, 0.26
+    crowded = usual.clone()
+    crowded[8], crowded[9] = 0.01, 0.02
+    wide = torch.linspace(-1.5, 1.5, 16)
+    for name, table in (("usual", usual), ("edge", edge), ("crowded", crowded), ("wide", wide)):
+        log(f"GPU quantiser, {name} table")
+        nf4 = table.cuda()
+        mid = (nf4[1:] + nf4[:-1]) * 0.5
+        g = torch.Generator(device="cuda")
+        g.manual_seed(5)
+        w = (torch.randn(3 * 16384, generator=g, device="cuda") * 0.02).half().view(-1, 64)
+        near = mid.half().repeat(4)[:60]
+        step = torch.tensor([-1, 0, 1, 2], dtype=torch.int16, device="cuda").repeat_interleave(15)
+        # (one step below the pattern of +0, a midpoint of the wide table, is no number: 0 there; the
+        # expected maximum below would be NaN, the kernel's skips it)
+        w[5, :60] = torch.nan_to_num((near.view(torch.int16) + step).view(torch.float16), nan=0.0)
+        w[5, 60:] = torch.tensor([1.0, -1.0, 0.0, -0.0], device="cuda").half()
+        packed = torch.empty(w.numel() // 2, dtype=torch.uint8, device="cuda")
+        rest = [torch.empty(w.numel() // n, dtype=dt, device="cuda")
+                for n, dt in ((64, torch.uint8), (16384, torch.float32), (16384, torch.float32))]
+        absmax, _ = quant.quantize_into(w.view(-1), code2, nf4, packed, *rest)
+        amax = w.float().abs().amax(1)
+        assert torch.equal(absmax, amax)
+        x = w.float() * (1.0 / amax)[:, None]
+        code = (x[:, :, None] > mid).sum(2).to(torch.uint8).view(-1, 2)
+        assert torch.equal(packed, (code[:, 0] << 4) | code[:, 1]), name
