@@ -118,3 +118,59 @@ def test_streamed_head_full_vocabulary(torch):
     s = float(np.abs(ref_dy).max()) or 1.0
     assert_close(host(dy).astype(np.float64) / s, ref_dy / s, 1e-2, 2e-2, "d(hidden)")
     assert not np.any(host(dy)[tgt < 0]), "rows without a target get a zero gradient"
+
+
+@pytest.mark.parametrize("vc", [8, 2040, 2048, 8184, 8192, 8200, 10248])
+def test_chunk_rows(torch, vc):
+    """The row kernel alone at the edges of its strides (256 threads x 8 columns x 4 pieces), with
+    ties, infinite logits, rows of -inf and a NaN.  The sums' bound: vc / 512 + 24 roundings (a
+    thread's two chains, then the lanes' and waves' sums), 2 ulp per exponential, and z's own
+    rounding, |z| 2^-24 of e^z with |z| under 26 where it counts; P is a rounding to fp16 of values
+    within that of the exact ones."""
+    from decentrik_prime_amd import _lib
+    lib = _lib.lib()
+    rng = np.random.default_rng(vc)
+    n, n_lab, d, v0, scale = 12, 9, 64, 40, 64.0
+    x = (rng.standard_normal((n, vc)) * 3).astype(np.float16)
+    top = x.max(1)
+    x[1, [vc // 2, vc - 1]] = top[1] + np.float16(1)            # a tie: the first counts
+    x[2, : vc // 2] = -np.inf
+    x[3] = -np.inf
+    x[3, vc - 3] = -5.0
+    x[4] = np.float16(-60000.0)                                 # far from the maximum: e^z is 0
+    x[4, 5] = 60000.0
+    x[5] = np.float16(2.0)                                      # all equal
+    x[11, 3] = np.nan
+    tgt = rng.integers(v0, v0 + vc, n).astype(np.int32)
+    tgt[6], tgt[7] = v0 - 1, v0 + vc                            # outside the chunk
+    tgt[9:] = -1
+    lg, st = torch.from_numpy(x).cuda(), torch.zeros(n, 8, device="cuda")
+    st[:, 0] = float("-inf")
+    acc = torch.ones(n, d, device="cuda")
+    t = torch.from_numpy(tgt).cuda()
+    log(f"head rows, {vc} columns")
+    rc = lib.dk_head_chunk(_lib.ptr(lg), _lib.ptr(t), _lib.ptr(st), _lib.ptr(acc), n, n_lab, vc, v0,
+                           scale, d, _lib.stream_handle(lg.device))
+    _lib.check(rc, "dk_head_chunk")
+    p, got = host(lg), host(st).astype(np.float64)
+    assert np.isnan(got[11, 1])
+    x64 = x[:11].astype(np.float64)
+    m = x64.max(1)
+    z = x64 - m[:, None]
+    ev = np.exp(z)
+    bound = (vc / 512 + 24 + 4 + 26) * 2.0 ** -24
+    assert np.array_equal(got[:11, 0], m) and np.array_equal(got[:11, 3], x64.argmax(1) + v0)
+    assert np.all(np.abs(got[:11, 1] - ev.sum(1)) <= bound * ev.sum(1)), "s"
+    ok = [r for r in range(11) if r not in (2, 3)]              # 0 x -inf there, as in the definition
+    tt = (ev[ok] * z[ok]).sum(1)
+    assert np.all(np.abs(got[ok, 2] - tt) <= bound * np.abs(tt) + 2.0 ** -120), "t"
+    assert np.isnan(got[2, 2]) and np.isnan(got[3, 2])
+    inside = (tgt[:11] >= v0) & (tgt[:11] < v0 + vc)
+    rows = np.nonzero(inside)[0]
+    assert np.array_equal(got[rows, 4], x64[rows, tgt[rows] - v0])
+    want = ev[:n_lab] * scale
+    for r in range(n_lab):
+        if inside[r]:
+            want[r, tgt[r] - v0] = 0.0
+    assert np.all(np.abs(p[:n_lab] - want) <= (2.0 ** -11 + 2.0 ** -18) * want + 2.0 ** -25), "P"
+    assert np.array_equal(p[n_lab:], x[n_lab:], equal_nan=True), "rows without a target stay"
