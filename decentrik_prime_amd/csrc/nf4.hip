@@ -1,7 +1,7 @@
 // NF4 double-quantised weights on gfx950: the HBM-rate dequant and the blockwise quantiser.
 //
 // Dequant (replaces solution/k_nf4.py:40-57).  Each wave converts one second-level block (2048
-// packed dwords of 8 weights, 16384 weights) with nf4_dev.h's dq_wave_load / dq_wave_store: every
+// packed dwords of 8 weights, 16384 weights), or a quarter of one where there are few, with nf4_dev.h's dq_wave_load / dq_wave_store: every
 // load instruction of the wave reads 256 contiguous bytes and every store instruction writes the
 // 64 lanes' 16-byte results, 1 KiB contiguous, straight from registers (no LDS staging, no
 // barrier before the stores).  A workgroup's four waves fill the two LDS tables (NF4 values and
@@ -10,13 +10,13 @@
 #include "nf4_dev.h"
 
 using dk::kWaveDwords;
-using dk::WaveLoads;
+using dk::WaveLoadsOf;
 using dk::dq_wave_load;
 using dk::dq_wave_store;
 
 namespace {
 
-// 32 dwords per lane (256 weights) in 256-thread workgroups, 714 per Qwen2.5-1.5B layer: measured
+// W = 32 dwords per lane (256 weights) in 256-thread workgroups, 714 per Qwen2.5-1.5B layer: measured
 // on MI355X over 28 layer buffers (graph-replayed, gaps included) 5.5-5.6 TB/s, against 4.8-5.0
 // for the former one-quad-per-lane kernel with LDS-staged stores, 5.1-5.2 for 8 or 16 dwords per
 // lane (16 with 512 threads), 4.8-5.1 for 8 or 16 with 1024 threads and 4.9 for 64; cached
@@ -24,9 +24,16 @@ namespace {
 // a plain copy of the packed words, 8 dwords per lane ran at the same 5.2 TB/s: more bytes in
 // flight per wave, not less arithmetic, is what raised the rate (writes alone reach 6.9 TB/s)
 constexpr int kDqThreads = 256;
-constexpr int kDqWgDwords = kDqThreads * kWaveDwords;
+// A weight that would not give every CU a workgroup of that form takes 8 dwords per lane, four times
+// as many workgroups: its time is one wave's chain of loads and stores, not the rate.  Measured
+// likewise on MI355X: [256, 1536] 6.8 -> 3.7 us, [1536, 1536] 7.5 -> 4.3 (16 dwords: 5.4),
+// [4096, 1536] 8.8 -> 6.1, [8960, 1536] 9.8 -> 8.8; beyond the line [11008, 2048] 12.5 against
+// 12.6 and [17920, 1536] 14.0 against 14.3.
+constexpr int kDqFew = 8;
+constexpr int64_t kDqFewMax = 256 * kDqThreads * kWaveDwords;   // dwords
 static_assert(kDqThreads == 256, "one code2 entry per thread");
 
+template <int W>
 __global__ __launch_bounds__(kDqThreads) void nf4_dequant_kernel(
     const uint32_t* __restrict__ packed, const uint8_t* __restrict__ qabs,
     const float* __restrict__ scale2, const float* __restrict__ offset2,
@@ -36,12 +43,12 @@ __global__ __launch_bounds__(kDqThreads) void nf4_dequant_kernel(
   __shared__ float c2[256];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t d_wave = (int64_t)blockIdx.x * kDqWgDwords + wave * 64 * kWaveDwords;
+  const int64_t d_wave = ((int64_t)blockIdx.x * kDqThreads + wave * 64) * W;
   const int64_t last = n_dwords - 1;
   // the tables' loads first (the LDS fill waits only for them), then the codes and the dwords
   const float c2v = code2[threadIdx.x];
   const float lutv = nf4[threadIdx.x & 15];
-  WaveLoads L;
+  WaveLoadsOf<W> L;
   dq_wave_load(packed, qabs, scale2, offset2, d_wave, last, lane, L);
   c2[threadIdx.x] = c2v;
   if (threadIdx.x < 16) lut[threadIdx.x] = lutv;
@@ -207,9 +214,12 @@ extern "C" int dk_nf4_dequant(const uint8_t* packed, const uint8_t* qabs, const 
   if (!packed || !qabs || !scale2 || !offset2 || !code2 || !nf4 || !out_f16) return DK_ERR_INVALID;
   if (!dk_aligned(packed, 16) || !dk_aligned(out_f16, 16)) return DK_ERR_ALIGN;
   const int64_t n_dwords = n_qblocks * 8;
-  const int64_t grid = (n_dwords + kDqWgDwords - 1) / kDqWgDwords;
+  const bool few = n_dwords <= kDqFewMax;
+  const int64_t per_wg = (int64_t)kDqThreads * (few ? kDqFew : kWaveDwords);
+  const int64_t grid = (n_dwords + per_wg - 1) / per_wg;
   if (grid > 0x7fffffff) return DK_ERR_INVALID;
-  hipLaunchKernelGGL(nf4_dequant_kernel, dim3((unsigned)grid), dim3(kDqThreads), 0, stream,
+  hipLaunchKernelGGL(few ? nf4_dequant_kernel<kDqFew> : nf4_dequant_kernel<kWaveDwords>,
+                     dim3((unsigned)grid), dim3(kDqThreads), 0, stream,
                      reinterpret_cast<const uint32_t*>(packed), qabs, scale2, offset2, code2, nf4,
                      reinterpret_cast<u32x4*>(out_f16), n_dwords);
   DK_CHECK_LAUNCH();

@@ -40,32 +40,35 @@ struct SideDequant {
   int wgs;
 };
 
-// One wave's share of a dequant: 64 lanes x kWaveDwords packed dwords (8 weights each) from dword
+// One wave's share of a dequant: 64 lanes x W (kWaveDwords) packed dwords (8 weights each) from dword
 // d_wave on, dword j of lane l at d_wave + 64 j + l, inside one second-level block (2048 dwords),
-// so scale2/offset2 are wave-uniform.  The wave spans 8 kWaveDwords first-level blocks: lane k
+// so scale2/offset2 are wave-uniform.  The wave spans 8 W first-level blocks: lane k
 // loads the codes of blocks k, k + 64, ... and forms their absmax once, and each dword takes its
 // block's absmax from the owning lane by a cross-lane read.  Every load goes out in
 // dq_wave_load, before any conversion; dq_wave_store converts and writes each dword's 8 fp16 as
 // one 16-byte store (the wave's store instruction writes 1 KiB contiguous).  Dwords past `last`
 // are loaded at clamped addresses and not stored.
 constexpr int kWaveDwords = 32;
-constexpr int kWaveOwn = kWaveDwords / 8;   // first-level codes per lane
 static_assert(64 * kWaveDwords <= DK_ELEMS_PER_SB / 8, "a wave within one second-level block");
 
-struct WaveLoads {
-  uint32_t w[kWaveDwords];
-  uint8_t q[kWaveOwn];
+template <int W = kWaveDwords>
+struct WaveLoadsOf {
+  static_assert(W % 8 == 0 && kWaveDwords % W == 0, "whole first-level codes per lane");
+  uint32_t w[W];
+  uint8_t q[W / 8];   // first-level codes of this lane
   float s2, o2;
 };
+using WaveLoads = WaveLoadsOf<>;
 
+template <int W>
 __device__ __forceinline__ void dq_wave_load(const uint32_t* __restrict__ packed,
                                              const uint8_t* __restrict__ qabs,
                                              const float* __restrict__ scale2,
                                              const float* __restrict__ offset2, int64_t d_wave,
-                                             int64_t last, int lane, WaveLoads& L) {
+                                             int64_t last, int lane, WaveLoadsOf<W>& L) {
   const int64_t blk_last = last / 8;
 #pragma unroll
-  for (int o = 0; o < kWaveOwn; ++o) {
+  for (int o = 0; o < W / 8; ++o) {
     const int64_t blk = d_wave / 8 + 64 * o + lane;
     L.q[o] = qabs[blk < blk_last ? blk : blk_last];
   }
@@ -73,22 +76,22 @@ __device__ __forceinline__ void dq_wave_load(const uint32_t* __restrict__ packed
   L.s2 = scale2[sb];
   L.o2 = offset2[sb];
 #pragma unroll
-  for (int j = 0; j < kWaveDwords; ++j) {
+  for (int j = 0; j < W; ++j) {
     const int64_t d = d_wave + 64 * j + lane;
     L.w[j] = __builtin_nontemporal_load(packed + (d < last ? d : last));
   }
 }
 
 // c2, lut: the 256-entry code table and the 16 NF4 values in LDS.  nt: non-temporal stores.
-template <bool NT>
-__device__ __forceinline__ void dq_wave_store(const WaveLoads& L, const float* c2, const float* lut,
+template <bool NT, int W>
+__device__ __forceinline__ void dq_wave_store(const WaveLoadsOf<W>& L, const float* c2, const float* lut,
                                               u32x4* __restrict__ out, int64_t d_wave,
                                               int64_t last, int lane) {
-  float amax_own[kWaveOwn];
+  float amax_own[W / 8];
 #pragma unroll
-  for (int o = 0; o < kWaveOwn; ++o) amax_own[o] = dk_absmax(c2[L.q[o]], L.s2, L.o2);
+  for (int o = 0; o < W / 8; ++o) amax_own[o] = dk_absmax(c2[L.q[o]], L.s2, L.o2);
 #pragma unroll
-  for (int j = 0; j < kWaveDwords; ++j) {
+  for (int j = 0; j < W; ++j) {
     // dword j of lane l is in block 8 j + l / 8 of the wave: lane (8 j + l / 8) % 64, entry 8 j / 64
     const float amax = __shfl(amax_own[j / 8], 8 * (j % 8) + (lane >> 3));
     const int64_t d = d_wave + 64 * j + lane;

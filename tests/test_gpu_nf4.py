@@ -54,6 +54,26 @@ def test_dequant_config0_bit_exact(torch_dev):
     assert np.array_equal(got, q["deq"].reshape(-1).view(np.uint16))
 
 
+@pytest.mark.parametrize("nq", [262143, 262144, 262145, 262144 + 700])
+def test_dequant_both_forms(torch_dev, nq):
+    """On both sides of the line (2^21 dwords, 262,144 blocks) between 8 and 32 dwords per lane,
+    every bit against the element rule."""
+    from decentrik_prime_amd import quant
+    log(f"dequant {nq} blocks")
+    rng = np.random.default_rng(nq)
+    n2 = -(-nq // 256)
+    g = {"packed": rng.integers(0, 256, nq * 32, dtype=np.uint8),
+         "qabs": rng.integers(0, 256, nq, dtype=np.uint8),
+         "scale2": rng.random(n2, dtype=np.float32), "offset2": rng.random(n2, dtype=np.float32),
+         "code2": rng.random(256, dtype=np.float32)}
+    nf4 = host(quant.nf4_table("cuda"))
+    sb = np.arange(nq) // 256
+    amax = g["code2"][g["qabs"]] * g["scale2"][sb] + g["offset2"][sb]
+    nib = np.stack([g["packed"] >> 4, g["packed"] & 15], 1).reshape(nq, 64)
+    want = (nf4[nib] * amax[:, None]).astype(np.float16)
+    assert np.array_equal(_dequant(torch_dev, g), want.reshape(-1).view(np.uint16))
+
+
 def test_dequant_range_leaves_the_rest(torch_dev):
     torch = torch_dev
     from decentrik_prime_amd import k_nf4, quant
