@@ -96,6 +96,8 @@ SIGNATURES = {
                                      _c_p, _i64, _c_p]),
     "dk_w4_linear_bwd_dx_lora": (_int, [_c_p, _i64, _i64, _W, _T, _int, _i64, _c_p, _i64, _int,
                                         _c_p, _i64, _c_p]),
+    "dk_w4_linear_bwd_lora": (_int, [_W, _c_p, _i64, _i64, ctypes.POINTER(LoraGradsTermC), _c_p,
+                                     _c_p, _i64, _int, _c_p, _i64, _c_p]),
     "dk_w4_linear_workspace": (_i64, [_i64, _W, _int]),
     "dk_w4_workspace": (_i64, [_i64, _W, _int]),
     "dk_h16_workspace": (_i64, [_i64, _i64, _i64, _int]),

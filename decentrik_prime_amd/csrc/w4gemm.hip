@@ -650,9 +650,10 @@ int launch_plan(const Plan& pl, GemmParams p, hipStream_t stream) {
 // (at least gemm_workspace bytes): split-K partials and, on the two-phase shapes, the weight
 // dequantised to fp16 in the workspace first (both launches on `stream`, in order).  The weight's
 // `kernel` field asks for the 256-tile kernel reading NF4 wherever its plan takes the shape (TILE).
-
+// LoRA column sums (sums->wgs > 0) join the GEMM of the second phase, which sets *carried.
 template <bool TRANS, int EPI>
-int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, hipStream_t stream) {
+int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, hipStream_t stream,
+             const SideSums* sums = nullptr, bool* carried = nullptr) {
   if (ws && ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
   // a few rows: every weight converted once, one launch, no workspace
   if constexpr (!TRANS) {
@@ -677,8 +678,13 @@ int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, h
                              w->rows * w->cols / DK_QBLOCK, stream))
     return e;
   p.w16 = w16;
+  if (sums) p.sums = *sums;
   const int big = hgemm_launch<TRANS, EPI>(p, ws, part_bytes, stream);
-  if (big != kHgemmDeclined) return big;
+  if (big != kHgemmDeclined) {
+    if (carried) *carried = true;
+    return big;
+  }
+  p.sums = SideSums{};
   return launch_plan<TRANS, EPI, true>(pl, p, stream);
 }
 
@@ -963,6 +969,35 @@ extern "C" int dk_w4_linear_bwd_dx(const void* dy, int64_t lddy, int64_t m,
   dk_lora_term t = {dz, lora_a, mask, 0, 0, keep_scale};
   return dk_w4_linear_bwd_dx_lora(dy, lddy, m, w, &t, dz ? 1 : 0, dz ? rank : 0, dx, lddx,
                                   out_mode, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dk_w4_linear_bwd_lora(const dk_nf4_weight* w, const void* x, int64_t m,
+                                     int64_t rank, const dk_lora_grads_term* term,
+                                     const void* lora_a, void* dx, int64_t lddx, int out_mode,
+                                     void* workspace, int64_t workspace_bytes,
+                                     hipStream_t stream) {
+  if (!weight_ok(w) || !term || !lora_a || term->n_out != w->rows) return DK_ERR_INVALID;
+  if (!dk_aligned(w->packed, 16)) return DK_ERR_ALIGN;
+  const dk_lora_term t = {term->dz, lora_a, term->mask, 0, 0, term->keep_scale};
+  GemmParams p = {};
+  if (int e = linear_bwd_params(p, term->dy, term->lddy, m, w->rows, w->cols, &t, 1, rank, dx, lddx,
+                                out_mode))
+    return e;
+  SideSums sums = {};
+  int blocks = 0;
+  if (int e = lora_sum_jobs(x, m, w->cols, rank, term, 1, &sums.jobs, &blocks)) return e;
+  if (int e = dk_lora_dz_multi(x, m, w->cols, rank, term, 1, stream)) return e;
+  bool carried = false;
+  if (m > 0) {
+    sums.rows = m;
+    sums.wgs = blocks;
+    set_weight(p, w);
+    const bool carry = rank == 16;
+    if (int e = dispatch<true, EPI_LINEAR>(p, w, workspace, workspace_bytes, stream,
+                                           carry ? &sums : nullptr, carry ? &carried : nullptr))
+      return e;
+  }
+  return carried ? 0 : lora_sums_launch(rank, sums.jobs, blocks, m, stream);
 }
 
 extern "C" int dk_w4_gateup_swiglu_fwd(const void* x, int64_t ldx, int64_t m,

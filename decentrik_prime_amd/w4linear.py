@@ -580,6 +580,39 @@ def lora_dz_multi(x, terms, outs=None):
     return LoraSums(x, arr, m, k, r, len(terms), keep, res)
 
 
+def _linear_backward_lora(dy, w, z, x, lora_A, lora_B, lora_scale=2.0, mask=None, keep_scale=1.0,
+                          out_dtype=torch.float32):
+    """(dX, dA, dB) of a linear with one adapter: lora_grads and linear_backward_dx in one call, bit
+    for bit, the column sums (dA, dB) carried by the dX GEMM where it has idle CUs for them."""
+    _check16(dy, "dy")
+    for t, nm in ((z, "z"), (x, "x"), (lora_A, "lora_A"), (lora_B, "lora_B")):
+        _check16(t, nm)
+        if not t.is_contiguous():
+            raise ValueError(f"{nm} must be contiguous")
+    m, n_out = dy.shape
+    r = z.shape[1]
+    if dy.shape[1] != w.rows:
+        raise ValueError(f"dy has {dy.shape[1]} columns, weight has {w.rows} rows")
+    if z.shape[0] != m or tuple(x.shape) != (m, w.cols) or tuple(lora_B.shape) != (n_out, r) \
+            or tuple(lora_A.shape) != (r, w.cols):
+        raise ValueError("linear_backward_lora: inconsistent shapes")
+    mask = _mask_ok(mask, (m, w.cols))
+    dev = dy.device
+    da = torch.empty(r, w.cols, dtype=torch.float32, device=dev)
+    db = torch.empty(n_out, r, dtype=torch.float32, device=dev)
+    dz = torch.empty(m, r, dtype=torch.float16, device=dev)
+    out, mode = _dx_out(None, m, w, out_dtype, False, dev)
+    term = _lib.LoraGradsTermC(_lib.ptr(dy), dy.stride(0), n_out, _lib.ptr(z), _lib.ptr(lora_B),
+                               float(lora_scale), _lib.ptr(mask), float(keep_scale), _lib.ptr(da),
+                               _lib.ptr(db), _lib.ptr(dz), None)
+    ws, nbytes = _workspace(w, m, _lib.DK_OP_LINEAR_BWD_DX, dev)
+    rc = _lib.lib().dk_w4_linear_bwd_lora(w.c_ref(), _lib.ptr(x), m, r, ctypes.byref(term),
+                                          _lib.ptr(lora_A), _lib.ptr(out), out.stride(0), mode,
+                                          _lib.ptr(ws), nbytes, _lib.stream_handle(dev))
+    _lib.check(rc, "dk_w4_linear_bwd_lora")
+    return out, da, db
+
+
 def gateup_swiglu_forward(x, w_gu, act=None, gu=None, save_gu=True, w16=None, side=None):
     """gate|up as one NF4 GEMM with the gated-SiLU epilogue.  w_gu is [2I, in] (gate rows then up
     rows).  Returns (act [M, I], gu [M, 2I] or None).  w16, side as in linear_forward_lora."""
@@ -661,9 +694,8 @@ class QLoRALinearFunction(torch.autograd.Function):
         x, z, a16, b16, mask = ctx.saved_tensors
         mask = mask if ctx.has_mask else None
         dy = dy.contiguous().half()
-        da, db, dz = lora_grads(dy, z, x, b16, ctx.s, mask, ctx.ks)
-        # in x's own dtype: the GEMM's one rounding of the fp32 sum, no fp32 copy of dx
-        dx = linear_backward_dx(dy, ctx.w, dz, a16, mask, ctx.ks, out_dtype=x.dtype)
+        # dx in x's own dtype: the GEMM's one rounding of the fp32 sum, no fp32 copy of dx
+        dx, da, db = _linear_backward_lora(dy, ctx.w, z, x, a16, b16, ctx.s, mask, ctx.ks, x.dtype)
         return (dx, da.to(ctx.dtypes[0]), db.to(ctx.dtypes[1]),
                 None, None, None, None, None)
 

@@ -351,6 +351,16 @@ typedef struct dk_side_lora_sums {
   int32_t n_terms;
 } dk_side_lora_sums;
 
+/* The whole backward of a linear with one LoRA adapter over an NF4 weight (n_out = w->rows,
+ * k = w->cols): dk_lora_grads' dz, dA and dB of `term` and dk_w4_linear_bwd_dx's dX with that dz,
+ * the term's mask and lora_a [rank, k], bit-identical to the two calls.  Where the GEMM runs on the
+ * dequantised weight with rank 16, its launch carries the column sums (dA, dB) on the CUs that its
+ * tiles leave idle.  workspace as for dk_w4_linear_bwd_dx. */
+int dk_w4_linear_bwd_lora(const dk_nf4_weight* w, const void* x, int64_t m, int64_t rank,
+                          const dk_lora_grads_term* term, const void* lora_a, void* dx,
+                          int64_t lddx, int out_mode, void* workspace, int64_t workspace_bytes,
+                          hipStream_t stream);
+
 /* gate|up as one NF4 GEMM with the gated-SiLU epilogue.  Replaces the gate and up GEMMs and
  * gated_silu_forward (solution/fast_qwen.py:1080-1108; solution/k_mlp.py:20-29):
  *   g = fp16(X Wg^T), u = fp16(X Wu^T), act = fp16(silu(g) * u)
