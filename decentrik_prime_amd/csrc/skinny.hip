@@ -60,11 +60,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void skinny_kernel(GemmParams p) {
     arow[t] = p.a + m * p.lda;
   }
   // slice c: K is a multiple of 64, so a lane's 64 weights lie inside K or past it; past it the
-  // last ones are read, and the A operand is zero
+  // last ones are read, and use() sets both operands to zero (in that one slice only)
   auto load = [&](int c, Slice<F16> (&sl)[CB], f16x8 (&a)[MT][8]) {
     const int64_t k0 = (int64_t)c * kSliceK + 64 * lg;
-    const bool in = k0 < K;
-    const int64_t k = in ? k0 : K - 64;
+    const int64_t k = k0 < K ? k0 : K - 64;
 #pragma unroll
     for (int b = 0; b < CB; ++b) {
       const int64_t e = wrow[b] + k;
@@ -84,18 +83,33 @@ __global__ __launch_bounds__(64 * kMaxWaves) void skinny_kernel(GemmParams p) {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const f16x8 v = *reinterpret_cast<const f16x8*>(arow[t] + k + 8 * j);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a[t][j][e] = in ? v[e] : (f16)0.0f;
-      }
+      for (int j = 0; j < 8; ++j) a[t][j] = *reinterpret_cast<const f16x8*>(arow[t] + k + 8 * j);
   };
   f32x4 acc[CB][MT];
 #pragma unroll
   for (int b = 0; b < CB; ++b)
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[b][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto use = [&](const Slice<F16> (&sl)[CB], const f16x8 (&a)[MT][8]) {
+  auto use = [&](int c, Slice<F16> (&sl)[CB], f16x8 (&a)[MT][8]) {
+    if ((c + 1) * (int64_t)kSliceK > K) {   // the last, partial slice: lanes past K add 0 * 0
+      const bool in = (int64_t)c * kSliceK + 64 * lg < K;
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          a[t][j] = in ? a[t][j] : f16x8{};
+#pragma unroll
+      for (int b = 0; b < CB; ++b) {
+        if constexpr (F16) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            sl[b].w[j] = in ? sl[b].w[j] : u32x4{0, 0, 0, 0};
+        } else {
+          sl[b].s2 = in ? sl[b].s2 : 0.0f;
+          sl[b].o2 = in ? sl[b].o2 : 0.0f;
+        }
+      }
+    }
 #pragma unroll
     for (int b = 0; b < CB; ++b) {
       const float amax = F16 ? 0.0f : dk_absmax(c2t[sl[b].code], sl[b].s2, sl[b].o2);
@@ -129,16 +143,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void skinny_kernel(GemmParams p) {
     __syncthreads();   // the tables are filled
     for (int c = wave; c < slices; c += 2 * ks) {
       if (c + ks < slices) load(c + ks, s1, a1);
-      use(s0, a0);
+      use(c, s0, a0);
       if (c + 2 * ks < slices) load(c + 2 * ks, s0, a0);
-      if (c + ks < slices) use(s1, a1);
+      if (c + ks < slices) use(c + ks, s1, a1);
     }
   } else {
     // two would not fit: the other waves hide the loads
     __syncthreads();
     for (int c = wave; c < slices; c += ks) {
       load(c, s0, a0);
-      use(s0, a0);
+      use(c, s0, a0);
     }
   }
 #pragma unroll

@@ -657,7 +657,10 @@ int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, h
   if (ws && ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
   // a few rows: every weight converted once, one launch, no workspace
   if constexpr (!TRANS) {
-    if (skinny_takes(p, EPI)) return skinny_launch<EPI, false>(p, stream);
+    if (skinny_takes(p, EPI)) {
+      if (ws && w->kernel != DK_W4_KERNEL_TILE && !dk_aligned(ws, 256)) return DK_ERR_ALIGN;
+      return skinny_launch<EPI, false>(p, stream);
+    }
   }
   // the 256-tile kernel with the weight dequantised in LDS, on request only (see two_phase)
   if (w->kernel == DK_W4_KERNEL_TILE) {
@@ -893,6 +896,14 @@ int dispatch_h16(GemmParams p, const void* w16, void* ws, int64_t ws_bytes,
   }
   if constexpr (!TRANS) {
     if (skinny_takes(p, EPI)) {   // no tiles to carry other work (NT GEMMs have no column sums)
+      // a workspace that the tiles would have refused is refused, though nothing here uses it
+      const int64_t own = plan_workspace(plan_for(p.M, p.N, p.K, EPI));
+      const int64_t tile = hgemm_workspace(p.M, p.N, p.K, EPI, true);
+      const int64_t need = tile >= 0 && tile < own ? tile : own;
+      if (ws && need > 0) {
+        if (ws_bytes < need) return DK_ERR_WORKSPACE;
+        if (!dk_aligned(ws, 256)) return DK_ERR_ALIGN;
+      }
       if (int e = skinny_launch<EPI, true>(p, stream)) return e;
       return side_alone(p.side, stream);
     }

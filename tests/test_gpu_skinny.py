@@ -85,3 +85,21 @@ def test_swiglu(torch, m, inter, d):
         return
     act16, gu16 = w4linear.gateup_swiglu_forward(x, w, w16=w.dequantize())
     assert torch.equal(act16, act) and torch.equal(gu16, gu), "NF4 and fp16 forms differ"
+
+
+@pytest.mark.parametrize("m", [1, 16, 20])
+@pytest.mark.parametrize("k", [64, 320, 512])
+def test_infinite_last_weight(torch, m, k):
+    """An infinite fp16 weight in the last 64 of K (which lanes past K read again) gives infinity."""
+    from decentrik_prime_amd import w4linear
+    log(f"skinny fp16 forward with an infinite weight {m} x 256 x {k}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + k)
+    w = _weight(torch, g, 256, k)
+    w16 = w.dequantize()
+    w16[5, k - 3] = float("inf")
+    x = (torch.rand(m, k, generator=g, device="cuda") + 0.5).half()
+    y = w4linear.linear_forward(x, w, w16=w16)
+    assert bool((y[:, 5] == float("inf")).all())
+    y[:, 5] = 0
+    assert bool(torch.isfinite(y).all())
