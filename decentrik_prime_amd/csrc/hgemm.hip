@@ -60,6 +60,7 @@ constexpr int kStageHalves = kTile * kBK;    // one operand of one stage: 32 KB
 constexpr int kEpiScratch = 16384;           // bytes of LDS per wave for the epilogue
 constexpr int kMidRows = 128;                // rows of a 128 x 256 tile
 constexpr int kMidStages = 3;
+constexpr int kQuarterRows = -1;             // GemmParams::xcd_gm: quarters over the rows of M alone
 constexpr int kMidHalves = kMidStages * (kMidRows + kTile) * kBK;   // its LDS: 144 KB
 static_assert(8 * kEpiScratch <= kMidHalves * 2, "epilogue scratch of a 128 x 256 tile");
 
@@ -1001,7 +1002,12 @@ void hgemm_kernel(GemmParams p, int main_tiles, int tail_wgs, int persist) {
   } else {
     int64_t m0, n0;
     const int t = b - qbase;
-    if (p.xcd_gm) {
+    if (p.xcd_gm == kQuarterRows) {
+      // an odd number of 128-row tiles, quarters only: none past M, M-fastest
+      const int tm = (int)((p.M + 127) / 128), u = xcd_run(t, tail_wgs);
+      m0 = 128 * (int64_t)(u % tm);
+      n0 = 128 * (int64_t)(u / tm);
+    } else if (p.xcd_gm) {
       // the quarters' parent tiles form a grid of tiles_m rows by the columns past the full tiles;
       // XCD x = t % 8 (workgroups are dealt to the XCDs round-robin) takes block (x % gm, x / gm)
       // of a gm x (8 / gm) split of that grid, so that its L2 holds the A rows and W rows of its
@@ -1227,7 +1233,9 @@ HPlan hplan_small(int64_t M, int64_t N, int64_t K, int epi, bool split, bool rop
     consider(plan_us(cost[COST_MID], tm2 * tn * s, cus, nk / s,
                      s > 1 ? tm2 * tn * s * kMidRows * kTile * 4 : 0),
              hplan_mid(M, N, s));
-  if (!rope) {
+  // w4gemm.hip's kernel: LINEAR only where the quarters leave half of the CUs idle (its unsplit tiles take
+  // far longer than the fit beyond: o forward at M = 2048 24.8 us against 17.7 as quarters)
+  if (!rope && (epi != EPI_LINEAR || 2 * tm2 * (N / 128) < cus)) {
     Plan st = plan_for(M, N, K, epi);
     if (!split) st.splits = 1;
     if (plan_us(cost[st.bn == 128 ? COST_STAGED128 : COST_STAGED64], st.tiles * st.splits, 2 * cus,
@@ -1235,6 +1243,18 @@ HPlan hplan_small(int64_t M, int64_t N, int64_t K, int epi, bool split, bool rop
       best.ok = false;
   }
   return best;
+}
+
+// One to two rounds of 256 x 256 tiles, or 128 x 256 tiles where those are estimated faster: they pad
+// an odd number of 128 rows by half a tile less (gate|up and down forward at M = 853 with the
+// dequants 110 -> 105 us).
+HPlan hplan_two(int64_t M, int64_t N, int64_t K, int epi, bool nt, int cus) {
+  const PlanCost* cost = kCost[epi == EPI_LINEAR ? (nt ? 0 : 1) : epi == EPI_SWIGLU_FWD ? 2 : 3];
+  const float nk = (float)(K / kBK);
+  const HPlan h = hplan_rounds(M, N, cus), mid = hplan_mid(M, N, 1);
+  const float t = plan_us(cost[COST_FULL], h.main_wgs, cus, nk, 0) +
+                  (h.tail_wgs ? plan_us(cost[COST_QUARTERS], h.tail_wgs, cus, nk, 0) : 0.0f);
+  return plan_us(cost[COST_MID], mid.main_wgs, cus, nk, 0) < t ? mid : h;
 }
 
 // w4: the plan of the NF4-reading form, which has no 128 x 256 tiles: where the fp16 form runs them
@@ -1246,12 +1266,20 @@ HPlan hplan(int64_t M, int64_t N, int64_t K, int epi, bool split, bool rope, boo
   if (cus <= 0) return h;
   const int64_t tiles = (M + kTile - 1) / kTile * (N / kTile);
   if (tiles * 4 > 0x7fffffff) return h;
-  h = tiles >= cus ? hplan_rounds(M, N, cus) : hplan_small(M, N, K, epi, split, rope, nt, cus);
+  h = tiles < cus ? hplan_small(M, N, K, epi, split, rope, nt, cus)
+      : tiles < 2 * cus && !w4 ? hplan_two(M, N, K, epi, nt, cus) : hplan_rounds(M, N, cus);
   if (w4 && h.ok && h.mid) {
     if (h.splits > 1) return HPlan{false, false, 0, 0, 0, 0, 1, 0};
     h = HPlan{true, false, (M + kTile - 1) / kTile, N / kTile, 0, 4 * tiles, 1, 0};
   }
-  if (h.ok && !h.mid && h.splits == 1)
+  // Quarters only, and an odd number of 128-row tiles: workgroups for the real ones alone.  With the
+  // empty ones of the last 256 rows in between, every other shader engine got more workgroups than
+  // CUs, hence a second round: N = 8960 at 257 to 384 rows 32 us where 256 rows took 18 (dX) and 33
+  // where they took 20 (SwiGLU backward); the MLP forward and backward at 300 to 320 rows 147 -> 131.
+  if (h.ok && !h.mid && h.splits == 1 && h.main_wgs == 0 && (M + 127) / 128 % 2 == 1) {
+    h.tail_wgs = (M + 127) / 128 * (N / 128);
+    h.xcd_gm = kQuarterRows;
+  } else if (h.ok && !h.mid && h.splits == 1)
     h.xcd_gm = xcd_blocks(h.tiles_m, h.main_wgs, h.tail_wgs,
                           epi == EPI_SWIGLU_BWD ? 0 : (int)h.main_wgs);
   return h;
@@ -1346,7 +1374,7 @@ int hgemm_launch(const GemmParams& p0, void* ws, int64_t ws_bytes, hipStream_t s
   const int cus = cu_count();
   const int persist = ((EPI == EPI_SWIGLU_FWD && h.main_wgs > cus) ||
                        (EPI == EPI_SWIGLU_BWD && h.tail_wgs > 0)) && !W4 && h.splits == 1 &&
-                      side == 0 && cus % 8 == 0 && h.main_wgs % 8 == 0 &&
+                      side == 0 && h.xcd_gm >= 0 && cus % 8 == 0 && h.main_wgs % 8 == 0 &&
                       (h.main_wgs / 8) % (cus / 8) == 0 && h.tail_wgs % 8 == 0 &&
                       h.tail_wgs / 8 <= cus / 8;
   hipLaunchKernelGGL((hgemm_kernel<TRANS, EPI, W4>),
