@@ -580,13 +580,25 @@ void w4_gemm_kernel(GemmParams p) {
 // 31.5 -> 24.5, q|k|v dX 42.3 -> 33.4.
 constexpr int64_t kTwoPhaseRows = 512;
 constexpr int64_t kTwoPhaseCols = 1536;
-
-//
 // Narrower outputs join them where the fp16 GEMM splits K.  (The 256-tile kernel can dequantise
 // the W tiles itself, bit-identically, but its per-step conversion costs more than the dequant
 // launch: gate|up dX at M = 853 82 + 10 us against 17 + 59 + 7.)
+//
+// Below kTwoPhaseRows the conversions of all row tiles decide: this file's kernel converts the
+// weight once per 128 rows, on workgroups that fill the CUs unevenly, so large weights gain from the
+// dequant launch as soon as they have a few row tiles.  Measured on MI355X, this file's kernel against
+// both launches: down forward at 257 to 384 rows 38 -> 31.5 us, gate|up forward at 400 to 511 61.5 ->
+// 50.5, gate|up dX at 257 62 -> 46, a [1536, 8960] weight's dX at 400 45 -> 39, the SwiGLU backward
+// at 129 44 -> 31 (at 33 even); on the other side of the lines down forward at 256 27.3 against 30,
+// gate|up forward at 384 42 against 49, an [8960, 1536] weight's forward at 400 43 against 44.
 bool two_phase(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
-  return M >= kTwoPhaseRows && (N >= kTwoPhaseCols || hgemm_workspace(M, N, K, epi, nt) > 0);
+  if (M >= kTwoPhaseRows) return N >= kTwoPhaseCols || hgemm_workspace(M, N, K, epi, nt) > 0;
+  if (N % 256 != 0) return false;   // hgemm.hip's kernels do not take it
+  const int64_t converted = (M + 127) / 128 * N * K;
+  if (epi == EPI_SWIGLU_BWD) return M > 32 && N * K >= (int64_t)4 << 20;
+  if (epi == EPI_SWIGLU_FWD) return converted >= (int64_t)100 << 20;
+  if (K >= N) return converted >= (int64_t)38 << 20;
+  return !nt && converted >= (int64_t)48 << 20;
 }
 
 int64_t round256(int64_t b) { return (b + 255) / 256 * 256; }
