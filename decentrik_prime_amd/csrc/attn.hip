@@ -266,19 +266,6 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int blk, int h,
   }
 }
 
-// 4 bytes per lane from global memory into LDS at lds + 4 * lane (the dword form of dma16).
-__device__ __forceinline__ void dma4(const void* src, unsigned lds) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %1\n\t"
-      "global_load_lds_dword %2, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "s"(lds), "v"(src)
-      : "memory");
-}
-
 // dK, dV per query head (solution/k_attn.py:97-139): one workgroup per (block of kBM keys, query
 // head), query tiles of kBN from the block's first key to the end of the sequence; fp32 partials
 // [N, NQ HD] that the QKV epilogue backward sums over each group of NQ / NKV heads.  The Q and dO

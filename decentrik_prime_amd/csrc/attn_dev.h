@@ -21,9 +21,15 @@
 // in the same order, read as columns of the row-major LDS tile by ds_read_b64_tr_b16 (the k order
 // of a product is free as long as both operands agree).  dK/dV compute S = Q K^T (the key on the
 // lane) and use P and dS the same way.
-#include "dk_common.h"
+#include "lds_dma.h"
 
 namespace {
+
+using dk::dma16s;
+using dk::dma4;
+using dk::lds_addr;
+using dk::uniform64;
+using dk::wait_vmem;
 
 constexpr int kHD = 128;          // head size (Qwen2.5: 128)
 constexpr int kAThreads = 256;    // 4 waves, 32 query rows (or keys) each
@@ -78,50 +84,6 @@ __device__ __forceinline__ int swz16(int r) {
 // offset (halves) of column c of row r in a swizzled tile
 __device__ __forceinline__ int sw_off(int r, int c) {
   return r * kHD + ((((c >> 3) ^ swz16(r))) << 3) + (c & 7);
-}
-
-__device__ __forceinline__ unsigned lds_addr(const void* p) {
-  return (unsigned)(size_t)(__attribute__((address_space(3))) const void*)p;
-}
-
-// 16 bytes per lane from global memory into LDS at lds + 16 * lane (inline assembly, so that the
-// compiler does not put a wait for it before every LDS read: the kernel counts these loads with
-// its own vmcnt waits; M0, the LDS address, is saved and restored around it).
-__device__ __forceinline__ void dma16(const void* src, unsigned lds) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %1\n\t"
-      "global_load_lds_dwordx4 %2, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "s"(lds), "v"(src)
-      : "memory");
-}
-
-// The same with a wave-uniform 64-bit base and a 32-bit byte offset per lane: one address register
-// per lane and no vector address arithmetic from tile to tile.
-__device__ __forceinline__ void dma16s(uint64_t base, unsigned off, unsigned lds) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %1\n\t"
-      "global_load_lds_dwordx4 %2, %3\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "s"(lds), "v"(off), "s"(base)
-      : "memory");
-}
-
-// A wave-uniform 64-bit value in scalar registers.
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) |
-         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)v);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 // Column (col + l % 32) of rows p .. p + 3 and p + 8 .. p + 11 of a swizzled tile, the 8 values of

@@ -47,6 +47,7 @@
 // of tiles (or a grid smaller than the CU count) leaves idle, and the dequant of the next layer's
 // weights runs under this GEMM instead of in a launch of its own.
 #include "gemm_common.h"
+#include "lds_dma.h"
 
 namespace dk {
 namespace {
@@ -67,42 +68,6 @@ static_assert(8 * kEpiScratch <= kMidHalves * 2, "epilogue scratch of a 128 x 25
 // Epilogue scratch of a wave with TN 32-column blocks per strip: the staged strip (32 rows of
 // 32 TN + 4 floats) plus the keep-mask and LoRA A slices (1536 bytes each).
 constexpr int epi_scratch_bytes(int tn) { return 32 * (32 * tn + 4) * 4 + 3072; }
-
-__device__ __forceinline__ unsigned lds_offset(const void* p) {
-  return (unsigned)(size_t)(__attribute__((address_space(3))) const void*)p;
-}
-
-// 16 bytes per lane from global memory into LDS at lds + 16 * lane.  Written as inline assembly
-// so that the compiler does not guard every later LDS read with a wait for it: the kernel tracks
-// these loads itself with vmcnt waits.  M0 (the LDS address) is saved and restored around it.
-// The SADDR form: the global address is a wave-uniform 64-bit base held in SGPRs plus a 32-bit
-// unsigned byte offset per lane.  One address register per lane instead of two and no per-load
-// address arithmetic (the base advances by whole K steps in scalar registers): in a
-// microbenchmark of the main loop on MI355X the loads cost 12.5 % of the MFMA issue cycles in
-// this form against 20 % with a 64-bit address per lane.
-__device__ __forceinline__ void dma16s(uint64_t base, unsigned off, unsigned lds) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %1\n\t"
-      "global_load_lds_dwordx4 %2, %3\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "s"(lds), "v"(off), "s"(base)
-      : "memory");
-}
-
-// A wave-uniform 64-bit value in scalar registers.  readfirstlane returns int: each half goes
-// through uint32_t so that the low half is zero-extended.
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) |
-         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((unsigned)v);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 __device__ __forceinline__ f16x4 read_tr(const f16* p) {
   return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -539,12 +504,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int64_t m0, int64
   auto issue = [&](int kt, int st, int d) {
     if (d < LA) {
       const unsigned dst = __builtin_amdgcn_readfirstlane(
-          lds_offset(As + st * SA + (d * NLW + lw) * 512));
+          lds_addr(As + st * SA + (d * NLW + lw) * 512));
       dma16s(a_base + (uint64_t)kt * (kBK * sizeof(f16)), a_off[d], dst);
     } else {
       const int j = d - LA;
       const unsigned dst = __builtin_amdgcn_readfirstlane(
-          lds_offset(Bs + st * SB + (j * NLW + lw) * 512));
+          lds_addr(Bs + st * SB + (j * NLW + lw) * 512));
       dma16s(b_base + (uint64_t)kt * b_step, b_off[j], dst);
     }
   };
