@@ -289,6 +289,7 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
   const bool nval = n < seqlen && s0 + n < a.n_tokens;
 
   const int n_tiles = (seqlen - nstart + kBN - 1) / kBN;   // at least 1 (block_of)
+  if ((int)threadIdx.x < kBN) lse_s[kBwdStages][threadIdx.x] = 0.0f;
   const TileSource qsrc = tile_source(a.qkv + (s0 + nstart) * ROW + (int64_t)h * kHD, ROW, wave, lane);
   const TileSource dsrc = tile_source(dout + (s0 + nstart) * OROW + (int64_t)h * kHD, OROW, wave, lane);
   // query tile t (queries nstart + 64 t ...); wave 0 also fetches the tile's lse, wave 1 its delta
@@ -348,6 +349,7 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
   };
   f16x8 fr[kAhead1];
   f32x4 ls[2], dl[2];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the row of zeros is written
   tile_barrier();
   f32x16 s_a[2], d_a[2], s_b[2], d_b[2];
   {
@@ -372,17 +374,27 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
     const int st = t % kBwdStages, m0 = nstart + t * kBN;
     // Keys past the sequence only reach rows of dK and dV that are not stored; queries before a
     // key or past the sequence are masked only on the tiles that hold such a query for this wave
-    // (a wave-uniform test): query q = m0 + off + 4 (l / 32) is kept iff lo <= off < hi; the
-    // others' probabilities come out as 0.
+    // (a wave-uniform test): query q = m0 + off + 4 (l / 32) is kept iff lo <= off < hi.  There the
+    // exponent is formed before the selection and the loop below is given scale 1 and a row of
+    // zeros for lse, so that the others' probabilities are 0 whatever their lse is: a NaN query
+    // reaches dV of no later key (masking the score alone would give e^NaN).
+    float scale = a.qk_scale;
+    int lrow = st;
     if (m0 < nstart + 32 * wave + 31 || m0 + kBN > seqlen) {
       const int lo = n - m0 - 4 * hl, hi = seqlen - m0 - 4 * hl;
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int g = 0; g < 8; ++g) {
+        const f32x4 l = g == 0 ? ls[0] : stat(lse_s, st, g);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int off = qb * 32 + 8 * (v >> 2) + (v & 3);
-          sc[qb][v] = ((off >= lo) & (off < hi)) ? sc[qb][v] : -1.0e30f;
+        for (int e = 0; e < 4; ++e) {
+          const int off = 8 * g + e;
+          const float x = __builtin_fmaf(sc[g >> 2][4 * (g & 3) + e], a.qk_scale, -l[e]);
+          sc[g >> 2][4 * (g & 3) + e] = ((off >= lo) & (off < hi)) ? x : -1.0e30f;
         }
+      }
+      scale = 1.0f;
+      lrow = kBwdStages;
+      ls[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     const unsigned nst = (unsigned)((t + 1) % kBwdStages) * kStageBytes;
     const unsigned qa = fresh(qrow + nst), da = fresh(drow + nst);
@@ -399,10 +411,10 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, int blk, int h,
       }
       const int qb = i >> 4, v = i & 15, g = i >> 2;
       if ((i & 3) == 0 && g + 1 < 8) {
-        ls[(g + 1) & 1] = stat(lse_s, st, g + 1);
+        ls[(g + 1) & 1] = stat(lse_s, lrow, g + 1);
         dl[(g + 1) & 1] = stat(dl_s, st, g + 1);
       }
-      sc[qb][v] = ex2(__builtin_fmaf(sc[qb][v], a.qk_scale, -ls[g & 1][i & 3]));
+      sc[qb][v] = ex2(__builtin_fmaf(sc[qb][v], scale, -ls[g & 1][i & 3]));
       dc[qb][v] = __fmul_rn(sc[qb][v], __fsub_rn(dc[qb][v], dl[g & 1][i & 3]));
       if (i & 1) {
         pf[i >> 3].h[(i >> 1) & 3] = pinned(sc[qb][v - 1], sc[qb][v]);
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(kAThreads) void attn_bwd_kernel(AttnArgs a, const f
   static_assert(kBwdStages == kFwdStages, "dK/dV and dQ share the tile ring");
   __shared__ __attribute__((aligned(1024))) f16 T0[kBwdStages * kTileHalves];
   __shared__ __attribute__((aligned(1024))) f16 T1[kBwdStages * kTileHalves];
-  __shared__ __attribute__((aligned(16))) float lse_s[kBwdStages][kBN], dl_s[kBwdStages][kBN];
+  __shared__ __attribute__((aligned(16))) float lse_s[kBwdStages + 1][kBN], dl_s[kBwdStages][kBN];
   const int per = n_blocks * a.nq;
   const int g = blockIdx.x;
   if (g < per)

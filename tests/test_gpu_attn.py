@@ -178,3 +178,39 @@ def test_table_entries_without_rows_are_skipped(torch):
     torch.cuda.synchronize()
     for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), *results):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"{name} changed"
+
+
+@pytest.mark.parametrize("t", [5, 70, 127, 150, 199])
+def test_bad_query_leaves_later_keys_alone(torch, t):
+    """A query that is NaN, or whose saved lse is, reaches dV of no later key (nor dK of one, with q
+    itself finite): those rows, and dQ of every other query, are bit for bit those of the clean
+    batch, in which the query's probabilities there are 0 as well."""
+    from decentrik_prime_amd import k_attn
+    lens = [37, 200, 64]
+    log(f"attention backward with a NaN at query {t}")
+    n, s0, nq, nkv = sum(lens), 37, 4, 2
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t)
+    qkv = (torch.randn(n, (nq + 2 * nkv) * HD, generator=g, device="cuda") * 0.8).half()
+    dout = torch.randn(n, nq * HD, generator=g, device="cuda").half()
+    meta = k_attn.meta_for(lens, "cuda")
+    out, lse = k_attn.attention_forward(qkv, meta, nq, nkv, HD)
+    clean = k_attn.attention_backward(qkv, out, lse, dout, meta, nq, nkv, HD)
+    others = torch.arange(n, device="cuda") != s0 + t
+    later = slice(s0 + t + 1, n)
+    for what in ("q", "lse"):
+        qkv2, lse2, out2 = qkv.clone(), lse.clone(), out
+        if what == "q":
+            qkv2[s0 + t, :nq * HD] = float("nan")
+            out2, lse2 = k_attn.attention_forward(qkv2, meta, nq, nkv, HD)
+            assert bool(torch.isnan(lse2[:, s0 + t]).all())
+            assert torch.equal(out2[others], out[others]), "out of the other queries"
+        else:
+            lse2[:, s0 + t] = float("nan")
+        dq, dk, dv = k_attn.attention_backward(qkv2, out2, lse2, dout, meta, nq, nkv, HD)
+        assert bool(torch.isnan(dv[s0: s0 + t + 1]).all()), "the keys that the query sees"
+        assert torch.equal(dq[others], clean[0][others]), f"{what}: dQ of the other queries"
+        assert torch.equal(dv[later], clean[2][later]), f"{what}: dV of later keys"
+        assert torch.equal(dv[:s0], clean[2][:s0]), f"{what}: dV of another sequence"
+        if what == "lse":
+            assert torch.equal(dk[later], clean[1][later]), f"{what}: dK of later keys"
