@@ -51,29 +51,15 @@ __device__ __forceinline__ int wg_min_int(int v, int* red) {
   return r;
 }
 
-// e^z for z <= 0 in seven instructions: 2^t on the hardware exponential at t = z log2(e) rounded, times
-// 1 + ln(2) d for the rounding d of t (the residual of the product, and z times the rest of
-// log2(e)).  Within 2 ulp of the exact value, as expf is (whose range and denormal handling took
-// twice the instructions); results below the normal range come out as 0.  e^-inf is 0 and e^NaN NaN:
-// fmaxf drops the rounding's own NaN (inf - inf).
-__device__ __forceinline__ float exp_le0(float z) {
-  constexpr float kL2E = 1.44269502162933349609375f;    // fp32(log2 e)
-  constexpr float kL2ELo = 1.92596299e-8f;              // log2 e - kL2E
-  constexpr float kLn2 = 0.693147182464599609375f;
-  const float t = __fmul_rn(z, kL2E);
-  const float d = fmaxf(__builtin_fmaf(z, kL2ELo, __builtin_fmaf(z, kL2E, -t)), -1.0f);
-  const float e = __builtin_amdgcn_exp2f(t);
-  return __builtin_fmaf(e, __fmul_rn(d, kLn2), e);
-}
-
 constexpr int kAhead = 4;   // pieces of a row in flight per thread
 
 // Bound: the row's logits from memory once (the second pass finds most of them in the caches) and P
-// back.  Before, 29 vector instructions per logit (a compare and two selects for the argmax, two for
-// the target's logit, expf) and one load in flight took longer.  Measured on MI355X, 32,768 columns:
-// 8 rows 20.9 -> 12.7 us, 853 rows 41.4 -> 32.6 (37.0 with expf), 2048 rows 70.6 -> 65.8.  Eight
-// pieces in flight or 512 threads a row were slower at 853 rows or at 4096 rows of 8192 columns.  The
-// sums' errors against 64 bits stay what they were (4.4e-8 of s rms, 1.5e-7 at most).
+// back.  Before, a compare and two selects per logit for the argmax, two for the target's logit and
+// one load in flight took longer.  Measured on MI355X, 32,768 columns (kernel trace): 8 rows 18.4 ->
+// 12.8 us, 853 rows 39.8 -> 36.0, 2048 rows 72.9 -> 71.9.  Eight pieces in flight or 512 threads a
+// row were slower at 853 rows or at 4096 rows of 8192 columns.  An exponential of half the
+// instructions (11.2, 31.7 and 67.2 us) is not used: its error, 0.59 x 2^-24 rms and 1.9 x 2^-24 at
+// most against expf's 0.44 and 1.4, and no results below 2^-126.
 __global__ __launch_bounds__(kHThreads) void head_chunk_kernel(
     f16* __restrict__ logits, const int32_t* __restrict__ tgt, float* __restrict__ state,
     float* __restrict__ acc, int64_t n_lab, int64_t vc, int64_t v0, float p_scale, int64_t d) {
@@ -135,7 +121,7 @@ __global__ __launch_bounds__(kHThreads) void head_chunk_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float z = __fsub_rn((float)x[e], mc);
-      const float ev = exp_le0(z);
+      const float ev = expf(z);
       as[e & 1] = __fadd_rn(as[e & 1], ev);
       at[e & 1] = __fadd_rn(at[e & 1], __fmul_rn(ev, z));
       p[e] = (f16)__fmul_rn(ev, pmul);

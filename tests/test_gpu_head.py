@@ -174,3 +174,24 @@ def test_chunk_rows(torch, vc):
             want[r, tgt[r] - v0] = 0.0
     assert np.all(np.abs(p[:n_lab] - want) <= (2.0 ** -11 + 2.0 ** -18) * want + 2.0 ** -25), "P"
     assert np.array_equal(p[n_lab:], x[n_lab:], equal_nan=True), "rows without a target stay"
+
+
+def test_chunk_rows_small_probabilities(torch):
+    """Probabilities below the normal range count: with a scale of 2^126 they come out in P.  e^z is
+    a multiple of 2^-149, half of which is the bound's last term; the first is P's own rounding and
+    2 ulp of e^z, the second half the smallest subnormal of fp16."""
+    from decentrik_prime_amd import _lib
+    lib = _lib.lib()
+    vc, scale = 4096, 2.0 ** 126
+    log("head rows, probabilities below the normal range")
+    x = np.zeros((1, vc), dtype=np.float16)
+    x[0, 1:] = -np.linspace(87.5, 102.0, vc - 1).astype(np.float16)
+    lg, st = torch.from_numpy(x).cuda(), torch.zeros(1, 8, device="cuda")
+    st[:, 0] = float("-inf")
+    acc, t = torch.zeros(1, 64, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(lib.dk_head_chunk(_lib.ptr(lg), _lib.ptr(t), _lib.ptr(st), _lib.ptr(acc), 1, 1, vc, 0,
+                                 scale, 64, _lib.stream_handle(lg.device)), "dk_head_chunk")
+    want = np.exp(x[0, 1:].astype(np.float64)) * scale
+    err = np.abs(host(lg)[0, 1:].astype(np.float64) - want)
+    bound = (2.0 ** -11 + 2.0 ** -22) * want + 2.0 ** -25 + 2.0 ** -149 * scale
+    assert np.all(err <= bound), float((err / want).max())
