@@ -1269,6 +1269,13 @@ int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
   return own > full ? own : full;
 }
 
+bool hgemm_scratch_optional(int64_t M, int64_t N, int64_t K, bool nt) {
+  if (M <= 0 || N % kTile || K % kBK || K < kBK) return false;
+  const int cus = cu_count();
+  if (cus <= 0) return false;
+  return (M + 127) / 128 * (N / 128) * 2 >= cus && (nt || M <= 3 * kTile || K < 4096);
+}
+
 // The epilogue writes 16-byte vectors of 8 consecutive columns.
 static bool vector_outputs_ok(const GemmParams& p, int epi) {
   if (epi == EPI_LINEAR)

@@ -1163,7 +1163,9 @@ extern "C" int dk_h16_linear_bwd_dx_lora_noalloc(const void* dy, int64_t lddy, i
   if (need > DK_NOALLOC_SCRATCH_BYTES) return DK_ERR_WORKSPACE;
   void* ws = nullptr;
   if (need > 0) {
-    if (int e = scratch_on_current_device(stream, &ws)) return e;
+    const int e = scratch_on_current_device(stream, &ws);
+    // captured before the array's address is known: unsplit where that will do
+    if (e && !(e == DK_ERR_CAPTURE && hgemm_scratch_optional(m, cols, rows, false))) return e;
   }
   return dispatch_h16<true, EPI_LINEAR>(p, w16, ws, ws ? DK_NOALLOC_SCRATCH_BYTES : 0, side,
                                         stream);

@@ -478,9 +478,11 @@ int dk_h16_linear_bwd_dx_lora_sums(const void* dy, int64_t lddy, int64_t m, cons
  * with a workspace of dk_h16_workspace bytes.  Every call on a device shares that device's array:
  * calls that overlap on one device (two streams, two threads) race and must be serialised by the
  * caller.  The array's device address is looked up (hipGetSymbolAddress) by the first call on
- * each device; under stream capture that first call returns DK_ERR_CAPTURE before doing anything,
- * so a caller that captures makes one call outside capture first (any later call, captured or
- * not, uses the address found then). */
+ * each device whose plan splits K; under stream capture that first call returns DK_ERR_CAPTURE
+ * before doing anything, so a caller that captures makes the same call once outside capture first
+ * (any later call, captured or not, uses the address found then).  A shape of at most 768 rows or
+ * with rows below 4096 whose 128 x 128 tiles fill half of the CUs is not refused there: that call
+ * runs without split K, bit-identical to dk_h16_linear_bwd_dx_lora with a NULL workspace. */
 #define DK_NOALLOC_SCRATCH_BYTES (64ll << 20)
 int dk_h16_linear_bwd_dx_lora_noalloc(const void* dy, int64_t lddy, int64_t m, const void* w16,
                                       int64_t rows, int64_t cols, const dk_lora_term* terms,

@@ -1,0 +1,75 @@
+"""The fp16-weight GEMM calls and their scratch memory: dk_h16_linear_bwd_dx_lora_noalloc under
+stream capture before the address of the library's scratch array is known."""
+
+import ctypes
+import shutil
+
+import pytest
+
+from tests.helpers import log
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    return t
+
+
+@pytest.mark.parametrize("m,rows,cols,refused", [
+    (390, 4096, 4096, False),      # 128 tiles of 128 x 128: half of the CUs
+    (768, 17920, 3072, False),     # 3 row tiles
+    (769, 17920, 3072, True),      # 4 row tiles and a long K: the scratch array
+    (260, 8960, 1536, True),       # 36 tiles of 128 x 128
+])
+def test_first_call_captured(torch, tmp_path, m, rows, cols, refused):
+    """A copy of the library, whose address look-up is still due, warmed up on a shape without split
+    K and then captured on one that the plan splits: refused, or run unsplit with the bits of the
+    call without a workspace, on every replay."""
+    from decentrik_prime_amd import _lib
+    path = tmp_path / "libdk_copy.so"
+    shutil.copy(_lib.LIB_PATH, path)
+    lib, name = ctypes.CDLL(str(path)), "dk_h16_linear_bwd_dx_lora_noalloc"
+    fn = getattr(lib, name)
+    fn.restype, fn.argtypes = _lib.SIGNATURES[name]
+    log(f"no-alloc dX captured as the first call that splits K: M={m} K={rows} N={cols}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    dy = (torch.randn(m, rows, device="cuda", generator=g) * 1e-2).half()
+    w = (torch.randn(rows, cols, device="cuda", generator=g) * 0.02).half()
+    out = torch.zeros(m, cols, dtype=torch.float16, device="cuda")
+    want = torch.empty_like(out)
+    _lib.check(_lib.lib().dk_h16_linear_bwd_dx_lora(
+        _lib.ptr(dy), rows, m, _lib.ptr(w), rows, cols, None, 0, 0, _lib.ptr(want), cols,
+        _lib.DK_OUT_F16, None, 0, None, _lib.stream_handle()), "without a workspace")
+    assert _lib.lib().dk_h16_workspace(m, rows, cols, _lib.DK_OP_LINEAR_BWD_DX) > 0
+
+    def call(rows_of_dy, k):
+        return fn(_lib.ptr(dy), rows, rows_of_dy, _lib.ptr(w), k, cols, None, 0, 0, _lib.ptr(out),
+                  cols, _lib.DK_OUT_F16, None, _lib.stream_handle())
+
+    warm = next(r for r in (m, 128, 64) if not _lib.lib().dk_h16_workspace(r, 64, cols, 1))
+    assert call(warm, 64) == 0
+    torch.cuda.synchronize()
+    out.zero_()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rc = call(m, rows)
+        if refused:
+            out.add_(1.0)     # (a graph of one node)
+    assert rc == (_lib.DK_ERR_CAPTURE if refused else 0)
+    for r in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        if refused:
+            assert bool((out == 1).all())
+        else:
+            assert torch.equal(out, want), f"replay {r}"
+    # outside capture the address is found, and the split plan runs
+    assert call(m, rows) == 0
+    ref = dy.double() @ w.double()
+    bound = rows * 2.0 ** -24 * (dy.double().abs() @ w.double().abs()) + 2.0 ** -11 * ref.abs() + 2.0 ** -25
+    assert bool(((out.double() - ref).abs() <= bound).all())
