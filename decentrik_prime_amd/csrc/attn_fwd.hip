@@ -29,11 +29,14 @@ __device__ __forceinline__ float half_max(float x) {
 __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __restrict__ out,
                                                              float* __restrict__ lse, int n_blocks) {
   // every head of a block before the next block, the table from its end: within a sequence the
-  // longest walks start first, so that no long block is left to run alone at the end
-  const int h = blockIdx.x % a.nq;
+  // longest walks start first, so that no long block is left to run alone at the end.  The grid is
+  // n_blocks x nq (one dimension of n_blocks nq workgroups would end at 2^32 work items, 699,050
+  // one-token sequences of 12 heads), its workgroups taken in launch order
+  const int g = (int)(blockIdx.y * (unsigned)n_blocks + blockIdx.x);
+  const int h = g % a.nq;
   int64_t s0;
   int seqlen, mstart;
-  if (!block_of(a, n_blocks - 1 - (int)blockIdx.x / a.nq, &s0, &seqlen, &mstart)) return;
+  if (!block_of(a, n_blocks - 1 - g / a.nq, &s0, &seqlen, &mstart)) return;
   const int lane = threadIdx.x & 63, hl = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int qw = wave & 3, kg = wave >> 2;   // query group, key-tile parity
@@ -303,8 +306,9 @@ extern "C" int dk_attn_fwd(const void* qkv, const int32_t* cu_seqlens, int32_t n
   if (n_blocks == 0) return 0;
   if (!out || !lse) return DK_ERR_INVALID;
   if (!dk_aligned(out, 16) || !dk_aligned(lse, 4)) return DK_ERR_ALIGN;
-  if ((int64_t)n_blocks * nq > INT32_MAX) return DK_ERR_INVALID;   // one workgroup index
-  hipLaunchKernelGGL(attn_fwd_kernel, dim3((unsigned)(n_blocks * nq)), dim3(kFThreads), 0,
+  // the workgroup's index (a token per block at the least: no device holds that many)
+  if ((int64_t)n_blocks * nq > INT32_MAX) return DK_ERR_INVALID;
+  hipLaunchKernelGGL(attn_fwd_kernel, dim3((unsigned)n_blocks, (unsigned)nq), dim3(kFThreads), 0,
                      stream, a, (f16*)out, lse, n_blocks);
   DK_CHECK_LAUNCH();
   return 0;

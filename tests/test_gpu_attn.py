@@ -93,6 +93,31 @@ def test_attention_head_configs(torch, nq, nkv):
     _close(host(dvp), dvp_ref, 3e-2, 2e-2, "dv per query head")
 
 
+def test_forward_of_many_short_sequences(torch):
+    """2^19 sequences of one token, 16 heads: more workgroups than one grid dimension holds (2^32
+    work items).  One key each: its value, and its score as lse."""
+    from decentrik_prime_amd import k_attn
+    n, nq, nkv = 1 << 19, 16, 1
+    log(f"attention fwd, {n} one-token sequences, {nq} query heads")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(19)
+    qkv = torch.randn(n, (nq + 2 * nkv) * HD, device="cuda", generator=g, dtype=torch.float16)
+    tab = torch.zeros(n, 2, dtype=torch.int32, device="cuda")
+    tab[:, 0] = torch.arange(n, dtype=torch.int32, device="cuda")
+    cu = torch.arange(n + 1, dtype=torch.int32, device="cuda")
+    meta = k_attn.AttnMeta(cu, tab.view(-1), tab.view(-1), n, n, n)
+    out, lse = k_attn.attention_forward(qkv, meta, nq, nkv, HD)
+    k, v = qkv[:, nq * HD:(nq + 1) * HD].double(), qkv[:, (nq + 1) * HD:]
+    assert all(torch.equal(out[:, h * HD:(h + 1) * HD], v) for h in range(nq))
+    scale = 1.4426950408889634 / HD ** 0.5
+    for h in range(nq):
+        qk = qkv[:, h * HD:(h + 1) * HD].double() * k
+        want = qk.sum(1) * scale
+        # the fp32 sum (HD 2^-24 of the products' magnitudes), and its scaling
+        lim = (HD + 2) * 2.0 ** -24 * qk.abs().sum(1) * scale
+        assert bool(((lse[h].double() - want).abs() <= lim).all())
+
+
 def test_attention_argument_checks(torch):
     from decentrik_prime_amd import k_attn
     meta = k_attn.meta_for([5, 7], "cuda")
