@@ -107,9 +107,10 @@ int skinny_launch(const GemmParams& p, hipStream_t stream);
 // Split-K partials the launch of that shape needs (0: no split; -1: the plan does not take the
 // shape); nt: NT (W stored [N][K]).
 int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt);
-// Whether a LINEAR GEMM splits K for speed alone: its 128 x 128 tiles fill half of the CUs, and (NN)
-// it has at most 3 row tiles of 256 or K below 4096.  Such a call does without scratch memory where
-// there is none to be had; the others ask for it.
-bool hgemm_scratch_optional(int64_t M, int64_t N, int64_t K, bool nt);
+// Split-K partials that a LINEAR GEMM which has a workspace must find room for: 0 where its 128 x 128
+// tiles fill half of the CUs and (NN) it has at most 3 row tiles of 256 or K below 4096, or with a 256 x 256
+// tile per CU (such a call splits K for speed alone, if it does: it runs without where there is no
+// scratch memory to be had); -1: w4gemm.hip's kernel decides.
+int64_t hgemm_required(int64_t M, int64_t N, int64_t K, bool nt);
 
 }  // namespace dk

@@ -1256,6 +1256,22 @@ int64_t partial_bytes(const HPlan& h) {
 
 }  // namespace
 
+int64_t hgemm_required(int64_t M, int64_t N, int64_t K, bool nt) {
+  if (M <= 0 || N % kTile || K % kBK || K < kBK) return -1;
+  const int cus = cu_count();
+  if (cus <= 0) return -1;
+  const int64_t tiles_m = (M + kTile - 1) / kTile, tiles = tiles_m * (N / kTile);
+  if (tiles * 4 > 0x7fffffff) return -1;
+  if (tiles >= cus) return 0;
+  const bool half = (M + 127) / 128 * (N / 128) * 2 >= cus;
+  if (tiles_m >= 4 && K >= 4096 && !(nt && half)) {
+    int64_t s = cus / tiles;
+    if (s > K / kBK / 8) s = K / kBK / 8;
+    if (s >= 2) return tiles * s * kTile * kTile * (int64_t)sizeof(float);
+  }
+  return half ? 0 : -1;
+}
+
 // Partials of the plan, or of the 256 x 256 tiles' own split over every CU where that is more (a
 // caller's buffer then holds either).
 int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
@@ -1267,13 +1283,6 @@ int64_t hgemm_workspace(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
   if (s > K / kBK / 8) s = K / kBK / 8;
   const int64_t own = partial_bytes(h), full = tiles * s * kTile * kTile * (int64_t)sizeof(float);
   return own > full ? own : full;
-}
-
-bool hgemm_scratch_optional(int64_t M, int64_t N, int64_t K, bool nt) {
-  if (M <= 0 || N % kTile || K % kBK || K < kBK) return false;
-  const int cus = cu_count();
-  if (cus <= 0) return false;
-  return (M + 127) / 128 * (N / 128) * 2 >= cus && (nt || M <= 3 * kTile || K < 4096);
 }
 
 // The epilogue writes 16-byte vectors of 8 consecutive columns.

@@ -906,16 +906,18 @@ int dispatch_h16(GemmParams p, const void* w16, void* ws, int64_t ws_bytes,
     p.sums.rows = sums.rows;
     p.sums.wgs = sums.blocks;
   }
+  // a given workspace that is too small for any of the plans below, or not aligned, is refused
+  // whichever of them runs
+  if (ws) {
+    int64_t need = plan_workspace(plan_for(p.M, p.N, p.K, EPI));
+    for (const int64_t t : {need > 0 ? hgemm_required(p.M, p.N, p.K, !TRANS) : 0,
+                            need > 0 ? hgemm_workspace(p.M, p.N, p.K, EPI, !TRANS) : 0})
+      if (t >= 0 && t < need) need = t;
+    if (need > 0 && ws_bytes < need) return DK_ERR_WORKSPACE;
+    if (need > 0 && !dk_aligned(ws, 256)) return DK_ERR_ALIGN;
+  }
   if constexpr (!TRANS) {
     if (skinny_takes(p, EPI)) {   // no tiles to carry other work (NT GEMMs have no column sums)
-      // a workspace that the tiles would have refused is refused, though nothing here uses it
-      const int64_t own = plan_workspace(plan_for(p.M, p.N, p.K, EPI));
-      const int64_t tile = hgemm_workspace(p.M, p.N, p.K, EPI, true);
-      const int64_t need = tile >= 0 && tile < own ? tile : own;
-      if (ws && need > 0) {
-        if (ws_bytes < need) return DK_ERR_WORKSPACE;
-        if (!dk_aligned(ws, 256)) return DK_ERR_ALIGN;
-      }
       if (int e = skinny_launch<EPI, true>(p, stream)) return e;
       return side_alone(p.side, stream);
     }
@@ -1165,7 +1167,7 @@ extern "C" int dk_h16_linear_bwd_dx_lora_noalloc(const void* dy, int64_t lddy, i
   if (need > 0) {
     const int e = scratch_on_current_device(stream, &ws);
     // captured before the array's address is known: unsplit where that will do
-    if (e && !(e == DK_ERR_CAPTURE && hgemm_scratch_optional(m, cols, rows, false))) return e;
+    if (e && !(e == DK_ERR_CAPTURE && hgemm_required(m, cols, rows, false) == 0)) return e;
   }
   return dispatch_h16<true, EPI_LINEAR>(p, w16, ws, ws ? DK_NOALLOC_SCRATCH_BYTES : 0, side,
                                         stream);

@@ -1,5 +1,6 @@
 """The fp16-weight GEMM calls and their scratch memory: dk_h16_linear_bwd_dx_lora_noalloc under
-stream capture before the address of the library's scratch array is known."""
+stream capture before the address of the library's scratch array is known, and workspaces that are
+too small or not aligned."""
 
 import ctypes
 import shutil
@@ -73,3 +74,47 @@ def test_first_call_captured(torch, tmp_path, m, rows, cols, refused):
     ref = dy.double() @ w.double()
     bound = rows * 2.0 ** -24 * (dy.double().abs() @ w.double().abs()) + 2.0 ** -11 * ref.abs() + 2.0 ** -25
     assert bool(((out.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("op,m,rows,cols,need", [
+    # the 128-row kernel's partials, [tiles][splits][128][128 or 64] fp32, or fewer where the plan
+    # asks for fewer; 0: any workspace will do
+    (0, 128, 1536, 8960, 12 * 8 * 65536), (0, 16, 1536, 8960, 12 * 8 * 65536),
+    (0, 300, 1536, 1536, 72 * 3 * 32768), (1, 769, 17920, 3072, 168 * 5 * 65536),
+    (1, 390, 4096, 4096, 0), (0, 16, 16384, 4096, 0), (0, 2048, 1536, 8960, 0),
+])
+def test_refused_workspaces(torch, op, m, rows, cols, need):
+    """A workspace of fewer bytes, or one not on 256 bytes, is refused before any launch; one just
+    large enough is not."""
+    from decentrik_prime_amd import _lib
+    log(f"fp16-weight GEMM, op {op}, M={m} {rows} x {cols}: workspaces around {need} bytes")
+    lib = _lib.lib()
+    need = min(need, lib.dk_h16_workspace(m, rows, cols, op))
+    k, n = (cols, rows) if op == 0 else (rows, cols)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + rows)
+    x = (torch.randn(m, k, device="cuda", generator=g) * 1e-2).half()
+    w = (torch.randn(rows, cols, device="cuda", generator=g) * 0.02).half()
+    out = torch.zeros(m, n, dtype=torch.float16, device="cuda")
+    ws = torch.zeros(need + 512, dtype=torch.uint8, device="cuda")
+
+    def call(shift, nbytes):
+        common = (_lib.ptr(x), k, m, _lib.ptr(w), rows, cols)
+        end = (ws.data_ptr() + shift, nbytes, None, _lib.stream_handle())
+        if op == 0:
+            return lib.dk_h16_linear_fwd_lora(*common, None, None, 0, 0, _lib.ptr(out), n, *end)
+        return lib.dk_h16_linear_bwd_dx_lora(*common, None, 0, 0, _lib.ptr(out), n, _lib.DK_OUT_F16, *end)
+
+    assert ws.data_ptr() % 256 == 0
+    ref = x.double() @ (w.double().t() if op == 0 else w.double())
+    mag = x.double().abs() @ (w.double().abs().t() if op == 0 else w.double().abs())
+    bound = k * 2.0 ** -24 * mag + 2.0 ** -11 * ref.abs() + 2.0 ** -25
+    if need:
+        assert call(0, need - 1) == _lib.DK_ERR_WORKSPACE
+        assert call(16, need) == _lib.DK_ERR_ALIGN
+        torch.cuda.synchronize()
+        assert bool((out == 0).all())
+    for shift, nbytes in ((0, need),) if need else ((0, 1), (16, 256)):
+        out.zero_()
+        assert call(shift, nbytes) == 0
+        assert bool(((out.double() - ref).abs() <= bound).all())
