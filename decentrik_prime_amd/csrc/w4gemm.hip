@@ -667,12 +667,17 @@ template <bool TRANS, int EPI>
 int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, hipStream_t stream,
              const SideSums* sums = nullptr, bool* carried = nullptr) {
   if (ws && ws_bytes < gemm_workspace(p.M, p.N, p.K, EPI, !TRANS)) return DK_ERR_WORKSPACE;
+  // a workspace that is not aligned is refused, except with TILE where that kernel can do without
+  // (the SwiGLU GEMMs split no K: a K below 4096 stands for theirs)
+  if (ws && !dk_aligned(ws, 256)) {
+    const int64_t k = EPI == EPI_LINEAR ? p.K : kBK;
+    if (w->kernel != DK_W4_KERNEL_TILE || hgemm_required(p.M, p.N, k, !TRANS) != 0) return DK_ERR_ALIGN;
+    ws = nullptr;
+    ws_bytes = 0;
+  }
   // a few rows: every weight converted once, one launch, no workspace
   if constexpr (!TRANS) {
-    if (skinny_takes(p, EPI)) {
-      if (ws && w->kernel != DK_W4_KERNEL_TILE && !dk_aligned(ws, 256)) return DK_ERR_ALIGN;
-      return skinny_launch<EPI, false>(p, stream);
-    }
+    if (skinny_takes(p, EPI)) return skinny_launch<EPI, false>(p, stream);
   }
   // the 256-tile kernel with the weight dequantised in LDS, on request only (see two_phase)
   if (w->kernel == DK_W4_KERNEL_TILE) {
@@ -684,7 +689,6 @@ int dispatch(GemmParams p, const dk_nf4_weight* w, void* ws, int64_t ws_bytes, h
     pl.splits = 1;
     return launch_plan<TRANS, EPI, false>(pl, p, stream);
   }
-  if (!dk_aligned(ws, 256)) return DK_ERR_ALIGN;
   if (pl.splits > 1) p.part = reinterpret_cast<float*>(ws);
   if (!two_phase(p.M, p.N, p.K, EPI, !TRANS)) return launch_plan<TRANS, EPI, false>(pl, p, stream);
   const int64_t part_bytes = partials(p.M, p.N, p.K, EPI, !TRANS);

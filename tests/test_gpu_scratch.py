@@ -1,6 +1,6 @@
 """The fp16-weight GEMM calls and their scratch memory: dk_h16_linear_bwd_dx_lora_noalloc under
 stream capture before the address of the library's scratch array is known, and workspaces that are
-too small or not aligned."""
+too small or not aligned (those of the NF4 GEMMs too)."""
 
 import ctypes
 import shutil
@@ -118,3 +118,34 @@ def test_refused_workspaces(torch, op, m, rows, cols, need):
         out.zero_()
         assert call(shift, nbytes) == 0
         assert bool(((out.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,rows,cols,kernel,refused", [
+    (300, 1536, 1536, 1, True), (1025, 1536, 8960, 1, True), (16, 1536, 8960, 1, True),
+    (2048, 1536, 8960, 1, False),                    # TILE, 128 x 128 tiles that fill half of the CUs
+    (2048, 1536, 8960, 0, True), (16, 1536, 8960, 0, True), (300, 1536, 1536, 2, True),
+])
+def test_misaligned_nf4_workspaces(torch, m, rows, cols, kernel, refused):
+    """The NF4 forward with a workspace off by 16 bytes: refused, except by the tile kernel where it
+    has no use for one."""
+    from decentrik_prime_amd import _lib, quant, w4linear
+    log(f"NF4 GEMM, M={m} {rows} x {cols}, kernel {kernel}: a misaligned workspace")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + rows)
+    x = (torch.randn(m, cols, device="cuda", generator=g) * 1e-2).half()
+    w16 = (torch.randn(rows, cols, device="cuda", generator=g) * 0.02).half()
+    w = w4linear.W4.from_params(quant.quantize_4bit(w16)).with_kernel(kernel)
+    y = torch.zeros(m, rows, dtype=torch.float16, device="cuda")
+    nbytes = max(256, _lib.lib().dk_w4_workspace(m, w.c_ref(), _lib.DK_OP_LINEAR_FWD))
+    ws = torch.zeros(nbytes + 256, dtype=torch.uint8, device="cuda")
+    rc = _lib.lib().dk_w4_linear_fwd(_lib.ptr(x), cols, m, w.c_ref(), None, None, None, 0, 1.0,
+                                     _lib.ptr(y), rows, ws.data_ptr() + 16, nbytes, _lib.stream_handle())
+    torch.cuda.synchronize()
+    if refused:
+        assert rc == _lib.DK_ERR_ALIGN and bool((y == 0).all())
+        return
+    assert rc == 0
+    d = w.dequantize().view(rows, cols).double()
+    ref = x.double() @ d.t()
+    bound = cols * 2.0 ** -24 * (x.double().abs() @ d.abs().t()) + 2.0 ** -11 * ref.abs() + 2.0 ** -25
+    assert bool(((y.double() - ref).abs() <= bound).all())
