@@ -93,6 +93,54 @@ def test_attention_head_configs(torch, nq, nkv):
     _close(host(dvp), dvp_ref, 3e-2, 2e-2, "dv per query head")
 
 
+@pytest.mark.parametrize("lens", [[1089, 2049], [1153, 1100], [2112]])
+def test_long_sequences(torch, lens):
+    """Sequences whose walks go round the tile rings several times, with even and odd numbers of
+    64-row tiles and a last tile of one row, 12 or all 64: every element against float64."""
+    from decentrik_prime_amd import k_attn
+    nq, nkv = 4, 2
+    log(f"attention fwd+bwd, {nq} / {nkv} heads, lens {lens}")
+    n, sm = sum(lens), HD ** -0.5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    qkv = (torch.randn(n, (nq + 2 * nkv) * HD, device="cuda", generator=g) * 0.8).half()
+    dout = torch.randn(n, nq * HD, device="cuda", generator=g).half()
+    meta = k_attn.meta_for(lens, "cuda")
+    out, lse = k_attn.attention_forward(qkv, meta, nq, nkv, HD)
+    got = k_attn.attention_backward(qkv, out, lse, dout, meta, nq, nkv, HD)
+
+    def near(a, want, lim, what):
+        over = (a.double() - want).abs() - lim
+        assert bool((over <= 0).all()), f"{what}: {int((over > 0).sum())} outside, worst {float(over.max())}"
+
+    s0 = 0
+    for L in lens:
+        rows = slice(s0, s0 + L)
+        s0 += L
+        for h in range(nq):
+            cols, kv = slice(h * HD, (h + 1) * HD), h // (nq // nkv)
+            q = qkv[rows, cols].double()
+            k = qkv[rows, (nq + kv) * HD:(nq + kv + 1) * HD].double()
+            v = qkv[rows, (nq + nkv + kv) * HD:(nq + nkv + kv + 1) * HD].double()
+            o, do = out[rows, cols].double(), dout[rows, cols].double()
+            sc = torch.where(torch.ones(L, L, device="cuda").tril() > 0, sm * (q @ k.t()), -float("inf"))
+            p = torch.softmax(sc, 1)
+            ds = p * (do @ v.t() - (o * do).sum(1, keepdim=True))
+            what = f"length {L}, head {h}: "
+            # 2^-10 of the magnitudes summed: the rounding of P and dS to fp16 (2^-11) and, under
+            # 2^-12, what the scores' fp32 sums (HD 2^-24 of their products) move P by and the fp32
+            # sums over up to 2112 keys; 2^-25 for values below fp16's normal range
+            near(out[rows, cols], p @ v, 2.0 ** -10 * (p @ v.abs()) + 2.0 ** -11 * o.abs() + 2.0 ** -24,
+                 what + "out")
+            near(lse[h, rows], torch.logsumexp(sc, 1) / 0.6931471805599453, 2.0 ** -12, what + "lse")
+            eds = 2.0 ** -10 * ds.abs() + 2.0 ** -25 + HD * 2.0 ** -23 * p * (
+                do.abs() @ v.abs().t() + (o * do).abs().sum(1, keepdim=True))
+            near(got[0][rows, cols], sm * (ds @ k), sm * (eds.tril() @ k.abs()), what + "dq")
+            near(got[1][rows, cols], sm * (ds.t() @ q), sm * (eds.tril().t() @ q.abs()), what + "dk")
+            near(got[2][rows, cols], p.t() @ do,
+                 (2.0 ** -10 * p + 2.0 ** -25).tril().t() @ do.abs(), what + "dv")
+
+
 def test_forward_of_many_short_sequences(torch):
     """2^19 sequences of one token, 16 heads: more workgroups than one grid dimension holds (2^32
     work items).  One key each: its value, and its score as lse."""

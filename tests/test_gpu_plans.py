@@ -119,3 +119,39 @@ def test_rotary_small_rows(torch):
         y = w4linear.linear_forward_rope(x, _w4(torch, 2048, 1536), None, [], pos, cos, sin, 1792, w16=w)
         slack = 1536 * TINY * (x.double().abs() @ w.double().abs().T)
         _check(torch, y, x.double() @ w.double().T, slack, 1, f"rotary at position 0, M = {m}")
+
+
+@pytest.mark.parametrize("m", [17, 300, 853, 2048, 2049, 3333, 4096])
+def test_rotary_rows(torch, m):
+    """The rotary forward with bias, two LoRA terms and rotations of random positions, on 128 x 128
+    tiles and (2049 rows on) 128 x 256 ones, where a wave finds its head's other half in the scratch
+    of the wave beside it."""
+    from decentrik_prime_amd import w4linear
+    from oracle import rope
+    d, kv, hd = 1536, 256, 128
+    n, cols = d + 2 * kv, d + kv
+    log(f"rotary GEMM, M = {m}")
+    g, x, w = _inputs(torch, m, n, d, 7 * m)
+    bias = (torch.randn(n, generator=g, device="cuda") * 0.1).half()
+    z = [(torch.randn(m, 16, generator=g, device="cuda") * 0.5).half() for _ in range(2)]
+    b = [(torch.randn(k, 16, generator=g, device="cuda") * 0.05).half() for k in (d, kv)]
+    cos, sin = (torch.from_numpy(t).cuda() for t in rope.rope_tables(4096, hd))
+    pos = torch.randint(0, 4096, (m,), generator=g, device="cuda", dtype=torch.int32)
+    terms = [(z[0], b[0], 0, d, 2.0), (z[1], b[1], cols, n, 2.0)]
+    y = w4linear.linear_forward_rope(x, _w4(torch, n, d), bias, terms, pos, cos, sin, cols, w16=w)
+    base = x.double() @ w.double().t() + bias.double()
+    lo = torch.zeros_like(base)
+    lo[:, :d] = z[0].double() @ b[0].double().t()
+    lo[:, cols:] = z[1].double() @ b[1].double().t()
+    # before the rotation: the fp32 sum, its rounding and the LoRA product's
+    err = d * TINY * (x.double().abs() @ w.double().abs().t()) + U * (base.abs() + 2 * lo.abs())
+    v = base + 2 * lo
+    h = v[:, :cols].view(m, -1, hd)
+    c, s = cos[pos.long()].double()[:, None], sin[pos.long()].double()[:, None]
+    half = hd // 2
+    other = torch.cat([-h[..., half:], h[..., :half]], -1)
+    v = torch.cat([(h * c + other * s).reshape(m, cols), v[:, cols:]], 1)
+    e = err[:, :cols].view(m, -1, hd)
+    turned = e * c.abs() + torch.cat([e[..., half:], e[..., :half]], -1) * s.abs() \
+        + 4 * TINY * (h.abs() + other.abs())
+    _check(torch, y, v, torch.cat([turned.reshape(m, cols), err[:, cols:]], 1), 1, "rotary y")
