@@ -65,11 +65,6 @@ __device__ __forceinline__ f32x16 mfma(const f16x8& a, const f16x8& b, const f32
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ f16x4 read_tr(const f16* q) {
-  return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) i16x4*)(q)));
-}
-
 // K / V (or Q / dO) tiles in a ring of LDS stages filled by LDS DMA (global_load_lds_dwordx4:
 // no registers, the next tiles' loads in flight while this one is computed on).  A tile is kBN
 // rows of 256 bytes with no padding; the 16-byte chunks of row r are permuted by swz16(r), so
@@ -86,18 +81,6 @@ __device__ __forceinline__ int sw_off(int r, int c) {
   return r * kHD + ((((c >> 3) ^ swz16(r))) << 3) + (c & 7);
 }
 
-// Column (col + l % 32) of rows p .. p + 3 and p + 8 .. p + 11 of a swizzled tile, the 8 values of
-// MFMA k index j = 0..7 for a lane half whose p = 16 t + 4 (l / 32).  ds_read_b64_tr_b16: within
-// a 16-lane group, lane 4a + b receives element b of the 4-half pieces addressed by lanes a,
-// a + 4, a + 8, a + 12; lane x addresses row p + x / 4 at columns col + 16 (group) + 4 (x % 4),
-// so lane x' of the group receives column col + 16 (group) + x' of the four rows.
-__device__ __forceinline__ f16x8 read_col8_sw(const f16* tile, int p, int col) {
-  const int lane = threadIdx.x & 63;
-  const int r = p + ((lane & 15) >> 2), c = col + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const f16x4 lo = read_tr(tile + sw_off(r, c)), hi = read_tr(tile + sw_off(r + 8, c));
-  return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-}
-
 // The operand reads of a tile by LDS byte address.  The swizzle only flips chunk bits, so every
 // operand of a tile is a lane's base address with a constant XORed into it (plus a constant row
 // offset): K operand of sub-step s of rows 0..31 (+ 32 rows: 8192 bytes on) at kaddr ^ 32 s, and
@@ -111,13 +94,18 @@ __device__ __forceinline__ f16x4 lds_read_tr(unsigned addr, int off) {
       (__attribute__((address_space(3))) i16x4*)((lds_char*)(size_t)addr + off)));
 }
 // this lane's base for lds_read8 (row c = lane % 32, columns 8 (lane / 32) .. + 7) and for
-// lds_read_tr (see read_col8_sw: rows 4 (lane / 32) + lane % 16 / 4)
+// lds_col8 (row 4 (lane / 32) + lane % 16 / 4, columns 16 (lane / 16 % 2) + 4 (lane % 4) .. + 3)
 __device__ __forceinline__ unsigned row_base(int lane) {
   return (unsigned)(sw_off(lane & 31, 8 * (lane >> 5)) * 2);
 }
 __device__ __forceinline__ unsigned col_base(int lane) {
   return (unsigned)(sw_off(4 * (lane >> 5) + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2);
 }
+// Column 32 hb + lane % 32 of rows p .. p + 3 and p + 8 .. p + 11 of a swizzled tile, p = 4 (lane / 32)
+// (+ off / 256 rows): the 8 values of MFMA k index j = 0..7.  ds_read_b64_tr_b16: within a 16-lane
+// group, lane 4a + b receives element b of the 4-half pieces addressed by lanes a, a + 4, a + 8,
+// a + 12; with lane x of the group at row p + x / 4, columns 4 (x % 4) .. + 3 of the group's 16, lane
+// x' receives column x' of the four rows.
 __device__ __forceinline__ f16x8 lds_col8(unsigned caddr, int hb, int off) {
   const f16x4 lo = lds_read_tr(caddr ^ (unsigned)(64 * hb), off);
   const f16x4 hi = lds_read_tr(caddr ^ (unsigned)(64 * (hb ^ 2)), off + 2048);

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kFThreads) void attn_fwd_kernel(AttnArgs a, f16* __
   // tile pair u (tiles 2 u, 2 u + 1; tiles past the last: none) of one operand into stages t % 4:
   // instruction i of wave w fills the stage's chunks (8 i + w) 64 + lane (rows past
   // the sequence read its last row: finite, and masked to p = 0).  A row's offset inside its
-  // tile fits 32 bits: the host refuses head counts whose rows reach 2^32 / 64 bytes.
+  // tile fits 32 bits: with nq <= 65535 (attn_args) a row is at most 50.4 MB, 64 rows 3.2 GB.
   const unsigned rowb = (unsigned)(ROW * (int64_t)sizeof(f16));
   const unsigned chunk = (unsigned)(((lane & 15) ^ swz16(4 * wave + (lane >> 4))) << 4);
   const unsigned off0 = (unsigned)(4 * wave + (lane >> 4)) * rowb + chunk;

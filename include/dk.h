@@ -235,12 +235,12 @@ int dk_w4_linear_fwd_lora(const void* x, int64_t ldx, int64_t m, const dk_nf4_we
 
 /* Workspace of the fused NF4 GEMMs.  No counterpart in the reference (cuBLAS manages its own);
  * it stands in for the reference's fp16 dequant workspace (solution/fast_qwen.py:398-418).
- * It holds split-K partial tiles and, from 512 rows on for outputs of at least 1536 columns (and
- * narrower ones whose fp16 GEMM splits K), the
- * weight dequantised to fp16 once per call (the "two-phase" path: dequant at HBM rate, then the
- * MFMA GEMM on fp16 W), which at many row tiles is faster than dequantising each W tile again for
- * every row tile.  Without a
- * workspace (NULL) every entry point still runs, in one phase with the dequant in LDS.
+ * It holds split-K partial tiles and, where that is faster, the weight dequantised to fp16 once per
+ * call (the "two-phase" path: dequant at HBM rate, then the MFMA GEMM on fp16 W, instead of
+ * dequantising each W tile again for every row tile).  Which shapes take it depends on the
+ * operation, the sizes and the device: this query alone says what a call needs, and a smaller
+ * workspace is DK_ERR_WORKSPACE.  Without a workspace (NULL) every entry point
+ * still runs, in one phase with the dequant in LDS.
  * Bytes needed at m rows for operation op (0: none). */
 #define DK_OP_LINEAR_FWD 0         /* dk_w4_linear_fwd, dk_w4_linear_fwd_lora */
 #define DK_OP_LINEAR_BWD_DX 1      /* dk_w4_linear_bwd_dx, dk_w4_linear_bwd_dx_lora */
