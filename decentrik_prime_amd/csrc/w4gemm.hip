@@ -580,9 +580,11 @@ void w4_gemm_kernel(GemmParams p) {
 // 31.5 -> 24.5, q|k|v dX 42.3 -> 33.4.
 constexpr int64_t kTwoPhaseRows = 512;
 constexpr int64_t kTwoPhaseCols = 1536;
-// Narrower outputs join them where the fp16 GEMM splits K.  (The 256-tile kernel can dequantise
-// the W tiles itself, bit-identically, but its per-step conversion costs more than the dequant
-// launch: gate|up dX at M = 853 82 + 10 us against 17 + 59 + 7.)
+// Narrower outputs join them past kTwoPhaseRows where the fp16 GEMM splits K, and dX past 768 rows
+// with K of 4096 or more in any case (N = 1024, K = 4096 at 2500 rows: this file's kernel 61.9 us, the
+// dequant and unsplit quarters 43.5; at 640 rows 28.0 against 30.9).  (The 256-tile kernel can
+// dequantise the W tiles itself, bit-identically, but its per-step conversion costs more than the
+// dequant launch: gate|up dX at M = 853 82 + 10 us against 17 + 59 + 7.)
 //
 // Below kTwoPhaseRows the conversions of all row tiles decide: this file's kernel converts the
 // weight once per 128 rows, on workgroups that fill the CUs unevenly, so large weights gain from the
@@ -591,14 +593,20 @@ constexpr int64_t kTwoPhaseCols = 1536;
 // 50.5, gate|up dX at 257 62 -> 46, a [1536, 8960] weight's dX at 400 45 -> 39, the SwiGLU backward
 // at 129 44 -> 31 (at 33 even); on the other side of the lines down forward at 256 27.3 against 30,
 // gate|up forward at 384 42 against 49, an [8960, 1536] weight's forward at 400 43 against 44.
+// One row tile is converted once either way, whatever the weight's size, and two gain only in dX with
+// K < N: 8192 x 8192 forward at 128 rows 43 us against 64, dX at one row 40 against 58, 3584 x
+// 18944 at 200 rows forward 70 against 75, dX 90 against 80.  A gate|up weight of 256 column tiles fills
+// the CUs with this file's kernel: 37888 x 3584 at 256 rows 131 against 157.
 bool two_phase(int64_t M, int64_t N, int64_t K, int epi, bool nt) {
-  if (M >= kTwoPhaseRows) return N >= kTwoPhaseCols || hgemm_workspace(M, N, K, epi, nt) > 0;
+  if (M >= kTwoPhaseRows && N >= kTwoPhaseCols) return true;
+  if (M > kTwoPhaseRows)
+    return (!nt && M > 768 && K >= 4096 && N % 256 == 0) || hgemm_workspace(M, N, K, epi, nt) > 0;
   if (N % 256 != 0) return false;   // hgemm.hip's kernels do not take it
-  const int64_t converted = (M + 127) / 128 * N * K;
+  const int64_t row_tiles = (M + 127) / 128, converted = row_tiles * N * K;
   if (epi == EPI_SWIGLU_BWD) return M > 32 && N * K >= (int64_t)4 << 20;
-  if (epi == EPI_SWIGLU_FWD) return converted >= (int64_t)100 << 20;
-  if (K >= N) return converted >= (int64_t)38 << 20;
-  return !nt && converted >= (int64_t)48 << 20;
+  if (epi == EPI_SWIGLU_FWD) return row_tiles > 1 && N < 256 * 128 && converted >= (int64_t)100 << 20;
+  if (K >= N) return row_tiles > 2 && converted >= (int64_t)38 << 20;
+  return !nt && row_tiles > 1 && converted >= (int64_t)48 << 20;
 }
 
 int64_t round256(int64_t b) { return (b + 255) / 256 * 256; }

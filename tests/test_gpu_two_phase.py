@@ -61,3 +61,29 @@ def test_swiglu(torch, m, inter, hidden):  # noqa: F811
         # 2^-20: the hardware exponential and reciprocal; near a zero of 1 + g (1 - sig) its terms count
         _check(torch, out, dact * coef, slack * coef.abs() + 2.0 ** -20 * (dact * ud).abs() * (1 + gd.abs())
                + 2.0 ** -20 * (dact * gd).abs(), 2, name)
+
+
+def test_which_calls_hold_a_copy(torch):  # noqa: F811
+    """The workspace holds the fp16 copy of the weight only where a launch of its own dequantises it:
+    never for one row tile of a linear or gate|up (converted once either way), nor for two with K >= N
+    or a gate|up weight that fills the CUs; dX into few columns past 512 rows does."""
+    import ctypes
+
+    from decentrik_prime_amd import _lib
+    fwd, dx, gu = _lib.DK_OP_LINEAR_FWD, _lib.DK_OP_LINEAR_BWD_DX, _lib.DK_OP_GATEUP_SWIGLU_FWD
+    t = torch.zeros(256, device="cuda")
+    for rows, cols, op, m, copy in (
+            (8192, 8192, fwd, 17, False), (8192, 8192, fwd, 128, False), (8192, 8192, dx, 1, False),
+            (8192, 8192, fwd, 256, False), (8192, 8192, fwd, 257, True), (3584, 18944, dx, 128, False),
+            (3584, 18944, dx, 129, True), (37888, 3584, gu, 128, False), (37888, 3584, gu, 384, False),
+            (28672, 4096, gu, 129, True), (4096, 1024, dx, 2500, True), (4096, 1024, dx, 512, False)):
+        # (the query reads the sizes alone)
+        c = _lib.NF4WeightC(*(t.data_ptr(),) * 6, rows, cols, _lib.DK_W4_KERNEL_AUTO)
+        need = _lib.lib().dk_w4_workspace(m, ctypes.byref(c), op)
+        small = _lib.lib().dk_h16_workspace(m, rows, cols, op) if op != gu else 0
+        assert (need >= small + 2 * rows * cols) == copy, (rows, cols, op, m, need, small)
+
+
+@pytest.mark.parametrize("m,rows,cols", [(128, 8192, 8192), (2500, 4096, 1024)])
+def test_linear_other_shapes(torch, m, rows, cols):  # noqa: F811
+    test_linear(torch, m, rows, cols)
