@@ -108,6 +108,18 @@ def test_swiglu_plans(torch, m, inter, d):
                + 2.0 ** -20 * (dact * gd).abs(), 2, name)
 
 
+@pytest.mark.parametrize("m,inter,d", [(3000, 768, 1536), (200, 9472, 3584), (1500, 2048, 1024)])
+def test_swiglu_on_mid_tiles(torch, m, inter, d):
+    """Unsplit 128 x 256 tiles where the quarters would take a second round."""
+    test_swiglu_plans(torch, m, inter, d)
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (1000, 1024, 1024), (2500, 1024, 4096)])
+def test_linear_near_ties(torch, m, n, k):
+    """Shapes where two plans are estimated alike."""
+    test_linear_plans(torch, m, n, k)
+
+
 def test_rotary_small_rows(torch):
     """The rotary forward has no split K: its rows and plans agree with the plain forward's columns."""
     from decentrik_prime_amd import w4linear
