@@ -98,8 +98,12 @@ constexpr int kHgemmDeclined = -1000;
 template <bool TRANS, int EPI, bool W4 = false>
 int hgemm_launch(const GemmParams& p, void* ws, int64_t ws_bytes, hipStream_t stream);
 // The NT GEMM of `p` for a few rows (skinny.hip), on packed NF4 weights or p.w16: up to 16 rows, or
-// 32 for a LINEAR weight of at most 2048 x 1536.
+// 32 for a LINEAR weight of at most 2048 x 1536.  Every 16 columns read all of A again, so large fp16
+// weights with K >= N are left to the tiles from 13 rows on, which split K over all CUs (16 rows:
+// 3584 x 18944 40.3 -> 35.2 us, 8192 x 8192 36.8 -> 33.7; at 12 rows 36.6 against 35.3, 33.7 against
+// 33.9 and 4096 x 14336 29.9 against 31.7).
 inline bool skinny_takes(const GemmParams& p, int epi) {
+  if (p.M > 12 && p.w16 && epi == EPI_LINEAR && p.K >= p.N && p.N * p.K >= (int64_t)48 << 20) return false;
   return p.M <= 16 || (p.M <= 32 && epi == EPI_LINEAR && p.N * p.K <= (int64_t)2048 * 1536);
 }
 template <int EPI, bool F16>

@@ -103,3 +103,18 @@ def test_infinite_last_weight(torch, m, k):
     assert bool((y[:, 5] == float("inf")).all())
     y[:, 5] = 0
     assert bool(torch.isfinite(y).all())
+
+
+@pytest.mark.parametrize("m", [12, 13, 16])
+def test_large_fp16_weight(torch, m):
+    """A large fp16 weight with K >= N: the few-row kernel up to 12 rows, tiles with split K beyond."""
+    from decentrik_prime_amd import w4linear
+    n, k = 4096, 14336
+    log(f"few rows, fp16 weight, {m} x {n} x {k}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    w16 = (torch.randn(n, k, generator=g, device="cuda") * 0.02).half()
+    w = _weight(torch, g, n, k)          # (only its shape matters beside w16)
+    slack = k * TINY * (x.double().abs() @ w16.double().abs().T)
+    _check(w4linear.linear_forward(x, w, w16=w16), x.double() @ w16.double().T, slack, 1, "y")
