@@ -79,6 +79,8 @@ __device__ __forceinline__ void tile_barrier() {
 // between the phases: after it, tile t - 1's stage takes tile t + 3, and tile t + 2 is readable.
 // The order is held by scheduling barriers: left to itself the compiler waited for each operand
 // read right before its MFMA.
+// Measured on MI355X with the delta launch, 12 query / 2 KV heads (graph replays): one sequence of
+// 8192 tokens 953 -> 741 us, of 2048 93.5 -> 70.8, 8 x 1024 186 -> 157, 4 x 512 41.3 -> 34.9.
 constexpr int kAhead1 = 6, kAhead2 = 4;
 
 // dQ (solution/k_attn.py:142-182): one workgroup per (block of kBM queries, query head), key
