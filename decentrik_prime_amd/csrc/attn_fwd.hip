@@ -17,7 +17,7 @@ namespace {
 // phase after every barrier.  So the scores of the wave's next tile are computed beside the
 // exponentials of the current one (S(t + 2) needs nothing of tile t), and the K ring runs a
 // pair of tiles ahead of the V ring.  Measured on MI355X, 12 query / 2 KV heads (graph replays): one
-// sequence of 8192 tokens 417 -> 257 us (535 TFLOP/s), of 2048 40.9 -> 36.8, 8 x 1024 73.6 -> 62.0,
+// sequence of 8192 tokens 417 -> 257 us (802 TFLOP/s), of 2048 40.9 -> 36.8, 8 x 1024 73.6 -> 62.0,
 // 4 x 512 16.6 as before.
 constexpr int kFThreads = 512;
 constexpr int kFLoads = kTileHalves / 8 / kFThreads;   // DMA instructions per operand per lane: 2
